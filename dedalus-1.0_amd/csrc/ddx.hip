@@ -15,6 +15,7 @@
 
 #include "../../include/ddx.h"
 #include "ddx_kernels.h"
+#include "ddx_mixed.h"
 #ifndef DDX_COL_XCD_GROUP
 #define DDX_COL_XCD_GROUP 1
 #endif
@@ -145,7 +146,10 @@ struct ddx_plan {
   long nk = 0;          // Ky*Kz*Kxp
   long npts = 0;        // nx*ny*nz
   long nref = 0;        // reference k elements
-  FftPlan fx, fy, fz;
+  FftPlan fx;
+  MixPlan my, mz;        // mixed-radix column passes
+  MixRow mx;             // mixed-radix x rows
+  bool mix_x = false;    // ... where the extent has a plan
   double* dkx = nullptr;
   double* dky = nullptr;
   double* dkz = nullptr;
@@ -331,13 +335,6 @@ long ws_field_stride(const ddx_plan* p) {
   return std::max(per, (long)p->nk);
 }
 
-int tile_width(int n, size_t cb) {
-  // two ping-pong tiles of n x W complex within 64 KiB of LDS
-  int W = 8;
-  while (W > 1 && (size_t)2 * n * W * cb > 65536) W /= 2;
-  return W;
-}
-
 // ---------------------------------------------------------------------------
 // column passes
 // ---------------------------------------------------------------------------
@@ -412,11 +409,7 @@ template <typename T>
 int launch_col(ddx_plan* p, ColArgs<T>& a, int nslabs, int nfields, int dir, bool spectral,
                int cat, int nsrc = 0) {
   if (nfields < 1 || nfields > DDX_MAXF) return fail(DDX_ERR_ARG, "bad field count");
-  a.W = tile_width(a.n, sizeof(cpx<T>));
-  const size_t lds = (size_t)2 * a.n * a.W * sizeof(cpx<T>);
-  if (lds > 65536) return fail(DDX_ERR_UNSUPPORTED, "column FFT too long for LDS");
-  dim3 grid((a.ncols + a.W - 1) / a.W, nslabs, nfields);
-  dim3 block(256);
+  if ((size_t)2 * a.n * sizeof(cpx<T>) > 65536) return fail(DDX_ERR_UNSUPPORTED, "column FFT too long for LDS");
   // algorithmic bytes: every valid input element read once, output written once
   const double per_in = (double)nslabs * a.in_rows * p->Kx;
   const double per_out = (double)nslabs * a.out_rows * p->Kx;
@@ -426,13 +419,9 @@ int launch_col(ddx_plan* p, ColArgs<T>& a, int nslabs, int nfields, int dir, boo
     LAUNCHCHK();
     return 0;
   }
-  if (dir > 0) {
-    if (spectral) hipLaunchKernelGGL((col_fft_kernel<T, 1, true>), grid, block, lds, p->stream, a);
-    else hipLaunchKernelGGL((col_fft_kernel<T, 1, false>), grid, block, lds, p->stream, a);
-  } else {
-    if (spectral) hipLaunchKernelGGL((col_fft_kernel<T, -1, true>), grid, block, lds, p->stream, a);
-    else hipLaunchKernelGGL((col_fft_kernel<T, -1, false>), grid, block, lds, p->stream, a);
-  }
+  const MixPlan& mp = a.n == p->my.n ? p->my : p->mz;
+  if (mp.n != a.n || !mix_col_launch<T>(p->stream, a, mp, nslabs, nfields, dir, spectral))
+    return fail(DDX_ERR_UNSUPPORTED, "column FFT array too large");
   LAUNCHCHK();
   return 0;
 }
@@ -450,7 +439,6 @@ void col_defaults(ColArgs<T>& a) {
 // Backward z pass (3D): compact (Ky, Kz, Kxp) -> (Ky, Nz, Kxp)
 template <typename T>
 void geom_bz(const ddx_plan* p, ColArgs<T>& a) {
-  a.fp = p->fz;
   a.tw = (const cpx<T>*)p->tw.at(p->az.n);
   a.n = p->az.n;
   a.in_rows = p->Kz; a.in_c = p->az.c;
@@ -468,7 +456,6 @@ void geom_bz(const ddx_plan* p, ColArgs<T>& a) {
 template <typename T>
 void geom_by(const ddx_plan* p, ColArgs<T>& a) {
   const long nz = p->az.n;
-  a.fp = p->fy;
   a.tw = (const cpx<T>*)p->tw.at(p->ay.n);
   a.n = p->ay.n;
   a.in_rows = p->Ky; a.in_c = p->ay.c;
@@ -486,7 +473,6 @@ void geom_by(const ddx_plan* p, ColArgs<T>& a) {
 template <typename T>
 void geom_fy(const ddx_plan* p, ColArgs<T>& a) {
   const long nz = p->az.n;
-  a.fp = p->fy;
   a.tw = (const cpx<T>*)p->tw.at(p->ay.n);
   a.n = p->ay.n;
   a.in_rows = p->ay.n; a.in_c = -1;
@@ -499,7 +485,6 @@ void geom_fy(const ddx_plan* p, ColArgs<T>& a) {
 // Forward z pass (3D): (Ky, Nz, Kxp) -> (Ky, Kz, Kxp)
 template <typename T>
 void geom_fz(const ddx_plan* p, ColArgs<T>& a) {
-  a.fp = p->fz;
   a.tw = (const cpx<T>*)p->tw.at(p->az.n);
   a.n = p->az.n;
   a.in_rows = p->az.n; a.in_c = -1;
@@ -621,6 +606,16 @@ int launch_row(ddx_plan* p, RowArgs<T>& a) {
   // the generic kernel stages whole rows of every field in LDS
   const int nseq = std::max((a.nin + 1) / 2, (a.nout + 1) / 2);
   const size_t lds = (size_t)2 * nseq * a.nx * sizeof(cpx<T>);
+  if (a.mode != ROW_PHYS && p->mix_x && (size_t)2 * a.nx * sizeof(cpx<T>) <= 65536) {
+    // plain fields run one per grid row, whatever their number
+    ProfScope prof(p, cat, bytes);
+    if (mix_row_launch<T>(p->stream, a, p->mx, nrows)) {
+      LAUNCHCHK();
+      return 0;
+    }
+    if (prof.a) p->evfree.push_back(prof.a);   // nothing launched: no record
+    prof.a = nullptr;
+  }
   if (lds > 65536 && a.mode != ROW_PHYS && std::max(a.nin, a.nout) > 1) {
     // several plain fields over the LDS of the generic kernel: one at a time
     const int nf = std::max(a.nin, a.nout);
@@ -635,7 +630,8 @@ int launch_row(ddx_plan* p, RowArgs<T>& a) {
   }
   if (lds > 65536) return fail(DDX_ERR_UNSUPPORTED, "x rows too long for LDS");
   ProfScope prof(p, cat, bytes);
-  hipLaunchKernelGGL((row_kernel<T>), dim3(nrows), dim3(256), lds, p->stream, a);
+  if (!(p->mix_x && mix_row_launch<T>(p->stream, a, p->mx, nrows)))
+    hipLaunchKernelGGL((row_kernel<T>), dim3(nrows), dim3(256), lds, p->stream, a);
   LAUNCHCHK();
   return 0;
 }
@@ -1447,11 +1443,15 @@ int plan_create(int ndim, const int64_t* xshape, const double* length, int preci
   }
   p->zfft = ndim == 3;
   p->nbatch = nbatch > 0 ? nbatch : 1;
-  if (make_fft_plan(p->ax.n, &p->fx) || make_fft_plan(p->ay.n, &p->fy) ||
-      make_fft_plan(p->zfft ? p->az.n : 1, &p->fz)) {
+  FftPlan fy, fz;
+  if (make_fft_plan(p->ax.n, &p->fx) || make_fft_plan(p->ay.n, &fy) || make_fft_plan(p->zfft ? p->az.n : 1, &fz)) {
     delete p;
     return fail(DDX_ERR_UNSUPPORTED, "grid extents must factor into 2, 3 and 5");
   }
+  // (extents beyond these plans are beyond the transforms' LDS bounds too)
+  p->mix_x = mix_row_plan(p->ax.n, &p->mx);
+  if (!mix_col_plan(p->ay.n, &p->my)) p->my.n = 0;
+  if (!mix_col_plan(p->zfft ? p->az.n : 1, &p->mz)) p->mz.n = 0;
   p->Kx = p->ax.K;
   p->Kxp = (p->Kx + 7) / 8 * 8;
   p->Ky = p->ay.K;

@@ -16,6 +16,20 @@ namespace ddx {
 
 #define DDX_MAXF 16
 
+// store, nontemporal (streaming) when nt is set (uniform per launch)
+template <typename T>
+__device__ __forceinline__ void st_nt(cpx<T>* p, cpx<T> v, bool nt) {
+  if (nt) {
+    typedef T v2 __attribute__((ext_vector_type(2)));
+    v2 w;
+    w.x = v.x;
+    w.y = v.y;
+    __builtin_nontemporal_store(w, reinterpret_cast<v2*>(p));
+  } else {
+    *p = v;
+  }
+}
+
 // One term of a derived field: coef * (i k_dim)^[dim >= 0] * source[src]
 struct Term {
   int src;
@@ -37,7 +51,6 @@ struct ColArgs {
   cpx<T>* out[DDX_MAXF];
   const cpx<T>* src[DDX_MAXF];  // sources for the spectral prologue
   Recipe rec[DDX_MAXF];
-  FftPlan fp;
   const cpx<T>* tw;
   const double* k_row;   // compact wavenumbers along the row axis (prologue)
   const double* k_slab;  // compact wavenumbers along the slab axis (prologue)
@@ -61,60 +74,37 @@ struct ColArgs {
   T scale;
 };
 
-template <typename T, int D, bool SPECTRAL>
-__global__ void __launch_bounds__(256) col_fft_kernel(const ColArgs<T> a) {
-  extern __shared__ unsigned char smem_raw[];
-  cpx<T>* A = reinterpret_cast<cpx<T>*>(smem_raw);
-  const int W = a.W, n = a.n;
-  cpx<T>* B = A + n * W;
-  const int f = blockIdx.z;
-  const long slab = blockIdx.y;
-  const int c0 = blockIdx.x * W;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-
-  for (int e = tid; e < n * W; e += nthr) {
-    const int m = e / W, c = e - m * W;
-    const int col = c0 + c;
-    cpx<T> v = mk(T(0), T(0));
-    if (col < a.ncols) {
-      int row;
-      if (a.in_c < 0) row = m;
-      else if (m <= a.in_c) row = m;
-      else if (m >= n - a.in_c) row = m - (n - a.in_rows);
-      else row = -1;
-      if (row >= 0) {
-        const long off = slab * a.in_ss + (long)row * a.in_rs + col;
-        if (SPECTRAL) {
-          const int nterm = a.rec[f].nterm;
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            if (t < nterm) {
-              const Term tm = a.rec[f].t[t];
-              cpx<T> x = a.src[tm.src][off];
-              if (tm.dim >= 0) {
-                const double kk = (tm.dim == 0) ? a.k_col[col]
-                                  : (tm.dim == a.row_dim ? a.k_row[row] : a.k_slab[slab]);
-                x = mul_is(x, T(kk));
-              }
-              v = v + scale(x, T(tm.coef));
-            }
-          }
-        } else {
-          v = a.in[f][off];
-        }
-      }
-    }
-    A[m * W + c] = v;
+// Field, column tile and slab of a workgroup of a column pass; false for the
+// padding of a 1D grid.
+template <typename T>
+__device__ __forceinline__ bool col_unit(const ColArgs<T>& a, int& f, int& tile, long& slab) {
+  if (a.xcd_group == 2) {
+    // Workgroups are dealt to the 8 XCDs round robin by linear index L.  XCD
+    // x = L mod 8 takes slabs x, x + 8, ..., and walks each slab tile by
+    // tile, the F fields of a tile one after another: fields that read the
+    // same sources (a spectral prologue) find them in that XCD's L2, and so
+    // do the lanes past the last column, which read the previous tile.
+    const long L = blockIdx.x, t = L >> 3;
+    const long per = (long)a.ntiles * a.nfields;
+    slab = (t / per) * 8 + (L & 7);
+    if (slab >= a.nslabs) return false;   // padding of the last group of 8 slabs
+    tile = (int)((t % per) / a.nfields);
+    f = (int)(t % a.nfields);
+  } else if (a.xcd_group) {
+    // L = 8 (floor(U / 8) F + f) + U mod 8 puts the F fields of unit
+    // U = (slab, tile) on one XCD, one after another
+    const long L = blockIdx.x, t = L >> 3;
+    const long U = (t / a.nfields) * 8 + (L & 7);
+    if (U >= (long)a.ntiles * a.nslabs) return false;   // padding of the last group
+    f = (int)(t % a.nfields);
+    tile = (int)(U % a.ntiles);
+    slab = U / a.ntiles;
+  } else {
+    f = blockIdx.z;
+    tile = blockIdx.x;
+    slab = blockIdx.y;
   }
-  __syncthreads();
-  cpx<T>* R = lds_fft<T, T, D>(A, B, a.fp, W, W, 1, true, a.tw, tid, nthr);
-  for (int e = tid; e < a.out_rows * W; e += nthr) {
-    const int j = e / W, c = e - j * W;
-    const int col = c0 + c;
-    if (col >= a.ncols) continue;
-    const int m = (a.out_c < 0 || j <= a.out_c) ? j : j + (n - a.out_rows);
-    a.out[f][slab * a.out_ss + (long)j * a.out_rs + col] = scale(R[m * W + c], a.scale);
-  }
+  return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -306,20 +296,6 @@ struct EpiArgs {
   const cpx<T>* tw_y;   // twiddles of length Ny (fused forward-y epilogue)
   int nt;               // nontemporal stores of deriv and upd_out
 };
-
-// store, nontemporal (streaming) when nt is set (uniform per launch)
-template <typename T>
-__device__ __forceinline__ void st_nt(cpx<T>* p, cpx<T> v, bool nt) {
-  if (nt) {
-    typedef T v2 __attribute__((ext_vector_type(2)));
-    v2 w;
-    w.x = v.x;
-    w.y = v.y;
-    __builtin_nontemporal_store(w, reinterpret_cast<v2*>(p));
-  } else {
-    *p = v;
-  }
-}
 
 template <typename T>
 __device__ inline void kvec(const KGeom& g, long idx, int& col, T& kx, T& ky, T& kz) {
@@ -904,7 +880,7 @@ __global__ void convert_kernel(const TI* in, TO* out, long n) {
   if (i < n) out[i] = TO(in[i]);
 }
 
-__global__ void twiddle_kernel(cpx<double>* tw, int n) {
+static __global__ void twiddle_kernel(cpx<double>* tw, int n) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   double s, c;
@@ -912,30 +888,30 @@ __global__ void twiddle_kernel(cpx<double>* tw, int n) {
   tw[j] = mk(c, -s);
 }
 
-__global__ void twiddle_f32_kernel(const cpx<double>* tw64, cpx<float>* tw32, int n) {
+static __global__ void twiddle_f32_kernel(const cpx<double>* tw64, cpx<float>* tw32, int n) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   tw32[j] = mk(float(tw64[j].x), float(tw64[j].y));
 }
 
-__global__ void zero_kernel(uint32_t* p, size_t nwords) {
+static __global__ void zero_kernel(uint32_t* p, size_t nwords) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (; i < nwords; i += stride) p[i] = 0u;
 }
 
-__global__ void copy16_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n) {
+static __global__ void copy16_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (; i < n; i += stride) dst[i] = src[i];
 }
 
-__global__ void copy1_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t n) {
+static __global__ void copy1_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t n) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[i];
 }
 
-__global__ void zero_bytes_kernel(uint8_t* p, size_t n) {
+static __global__ void zero_bytes_kernel(uint8_t* p, size_t n) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
 }

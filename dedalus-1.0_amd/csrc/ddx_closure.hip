@@ -165,6 +165,7 @@ __device__ inline bf16x4 lds4(const uint16_t* p) {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // eight consecutive bf16 from LDS as two 8-byte reads
 __device__ inline bf16x8 lds8(const uint16_t* p) {
@@ -951,7 +952,6 @@ template <int CI, int CO, int NT>
 struct NetStage {
   static constexpr int NCO = CO / 16, KQ = CI == 32 ? 8 : 4;
   static constexpr int NCH = 9 * NCO * 64, R = (NCH + NT - 1) / NT;
-  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
   typedef typename std::conditional<CI == 32, u32x4, u32x2>::type chunk;
   chunk c[R];
   float b[NCO][4];
@@ -1211,6 +1211,338 @@ int launch_net(const NetArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((conv_net_kernel<NL, HID, TX, TY, NT>), dim3((unsigned)ntiles), dim3(NT), lds, s, a);
   CL_LAUNCHCHK("conv_net");
   return 0;
+}
+
+// ---------------------------------------------------------------------------
+// The whole network, row by row
+// ---------------------------------------------------------------------------
+//
+// A workgroup runs all five layers over a strip of rows of one image, full
+// width W (32 or 64): at step t layer l computes row y0 - 4 + t - 3 l from
+// the three rows that layer l - 1 left in a ring of four rows in LDS.
+// Columns wrap inside the row, so only the strip's ends are recomputed (S + 8
+// rows of layer 0 for S outputs, ..., S of layer 4), where the tile kernel's
+// halo is 1.83 times the network's work.  A wavefront keeps one layer and one
+// 16-pixel fragment of the row for the whole strip, and its weights in
+// registers (72 for 32 x 32 channels), so LDS carries little but activations:
+// group 0 takes the first and the last layer (half a layer each; the last
+// one's weights are read from LDS in MFMA operand order, for which its
+// registers do not suffice), group g layer g; with W = 64 each SIMD holds one
+// wavefront of every group.
+//
+// A step issues the row's MFMAs interleaved with bias, GELU and rounding of
+// the row of the step before: the matrix pipe takes 16 cycles an MFMA and
+// the activations 1.5 times that in VALU cycles, and wavefronts that leave a
+// barrier together do not overlap the two by themselves.  That row is
+// written a step late, hence the lag of three rows per layer.  The loop is
+// unrolled over the four ring positions, which makes every LDS row an
+// immediate offset.
+//
+// What bounds it: VALU issue, about 2400 cycles of a step's 2700 at 2 GHz (8
+// activations of 14.5 issue slots per lane and wavefront, and the addresses).
+// 256 images 64^2: 213 us with the tile kernel, 1.83 times the network's
+// MFMAs; row by row 150 us with two fragments per wavefront and 8 wavefronts
+// per CU, 128 with one and 16, 112 with the last layer's weights in LDS (128
+// registers without spills).
+//
+// One 16-byte chunk q (8 channels) of pixel p lies at chunk q ^ ((p >> 2) & 3)
+// of the pixel's 64 bytes: the 16 pixels of a fragment read one chunk each
+// from 16 distinct bank groups, for any shift of the fragment.
+//
+// The arithmetic is conv_net_kernel's: the same products in the same order.
+// Rows before a layer's first and after its last are computed from whatever
+// the rings hold and never reach a row that is stored.
+template <int W>
+struct RowNet {
+  static constexpr int WPG = W / 16;                   // wavefronts per group
+  static constexpr int NT = 4 * WPG * 64;
+  static constexpr int HROW = W * 64, IROW = W * 32;   // bytes of a row: hidden, input
+  static constexpr int HB = 4 * HROW, IB = 4 * IROW;   // rings of four rows
+  static constexpr int WG_PER_CU = 1024 / NT;          // 128 registers: 16 wavefronts per CU
+  static constexpr int WB = 9 * 64 * 16;               // the last layer's weights
+  static constexpr int lds_bytes() { return IB + 4 * HB + WB; }
+};
+
+__device__ __forceinline__ int rn_off(int p, int q) { return p * 64 + ((q ^ (p >> 2)) & 3) * 16; }
+__device__ __forceinline__ int rn_ioff(int p, int h) { return p * 32 + ((h ^ (p >> 3)) & 1) * 8 + (h & 2) * 8; }
+
+// two fp32 -> packed bf16, round to nearest even (one v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t f2bf2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+template <int CI, int CO>
+struct RowWeights {
+  static constexpr int NCO = CO / 16, KQ = CI == 32 ? 8 : 4;
+  typedef typename std::conditional<CI == 32, bf16x8, bf16x4>::type frag;
+  frag w[9][NCO];
+  float b[NCO][4];
+  __device__ __forceinline__ void load(const uint16_t* wp, const float* bp, int lane) {
+    const int m = lane & 15, kq = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int j = 0; j < NCO; ++j) {
+        const uint16_t* q = wp + ((j * 16 + m) * 9 + t) * CI + kq * KQ;
+        if constexpr (CI == 32) w[t][j] = gld8(q);
+        else w[t][j] = __builtin_bit_cast(bf16x4, *reinterpret_cast<const u32x2*>(q));
+      }
+#pragma unroll
+    for (int j = 0; j < NCO; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[j][i] = bp[j * 16 + 4 * kq + i];
+  }
+};
+
+// One row of a layer at this wavefront's fragment: off[dx] the LDS offset of
+// the lane's operand, shifted by dx - 1, in ring slot 0; the three rows lie
+// in slots S0, S0 + 1, S0 + 2 (mod 4).
+template <int CI, int CO, int ROW, int S0>
+__device__ __forceinline__ void rn_conv(const unsigned char* lds, const int (&off)[3], const RowWeights<CI, CO>& wt,
+                                        f32x4 (&acc)[CO / 16]) {
+  constexpr int NCO = CO / 16;
+  constexpr int base[3] = {(S0 & 3) * ROW, ((S0 + 1) & 3) * ROW, ((S0 + 2) & 3) * ROW};
+#pragma unroll
+  for (int j = 0; j < NCO; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < 9; ++t) {
+    const uint16_t* p = reinterpret_cast<const uint16_t*>(lds + off[t % 3] + base[t / 3]);
+    if constexpr (CI == 32) {
+      const bf16x8 xv = lds16(p);
+#pragma unroll
+      for (int j = 0; j < NCO; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt.w[t][j], xv, acc[j], 0, 0, 0);
+    } else {
+      const bf16x4 xv = __builtin_bit_cast(bf16x4, *reinterpret_cast<const u32x2*>(p));
+#pragma unroll
+      for (int j = 0; j < NCO; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wt.w[t][j], xv, acc[j], 0, 0, 0);
+    }
+  }
+}
+
+// The last layer's row, its weights from LDS (chunk t 64 + lane)
+template <int ROW, int S0>
+__device__ __forceinline__ void rn_conv_last(const unsigned char* lds, const int (&off)[3], const unsigned char* wl,
+                                             f32x4& acc) {
+  constexpr int base[3] = {(S0 & 3) * ROW, ((S0 + 1) & 3) * ROW, ((S0 + 2) & 3) * ROW};
+  acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < 9; ++t) {
+    const bf16x8 xv = lds16(reinterpret_cast<const uint16_t*>(lds + off[t % 3] + base[t / 3]));
+    const bf16x8 wv = lds16(reinterpret_cast<const uint16_t*>(wl + t * 1024));
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, xv, acc, 0, 0, 0);
+  }
+}
+
+// Activations of a row, written to ring slot SLOT: out[j] the LDS offset of
+// the lane's four channels, output channels 16 j ..
+template <int CI, int ROW, int SLOT>
+__device__ __forceinline__ void rn_hidden(unsigned char* lds, const int (&out)[2], const RowWeights<CI, 32>& wt,
+                                          const f32x4 (&acc)[2]) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = gelu(acc[j][i] + wt.b[j][i]);
+    *reinterpret_cast<uint2*>(lds + out[j] + (SLOT & 3) * ROW) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+  }
+}
+
+// An input row y (wrapped), 32 bytes of 16 bf16 channels per pixel: thread
+// tid < 2 W of group 0 brings half tid & 1 of pixel tid >> 1
+template <int W, bool FIELDS>
+struct RowInput {
+  uint4 q;
+  __device__ __forceinline__ void load(const NetArgs& a, int b, int y, int tid) {
+    if (tid >= 2 * W) return;
+    const int p = tid >> 1, h = tid & 1;
+    const long gp = ((long)b * a.H + wrapm(y, a.H)) * W + p;
+    if (!FIELDS) {
+      q = *reinterpret_cast<const uint4*>(&a.x[gp * 16 + 8 * h]);
+    } else {
+      float v[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const int ch = 8 * h + c, cc = ch < a.cin ? ch : 0;
+        v[c] = ch < a.cin ? (float)a.src[cc][gp] * a.in_scale[cc] : 0.f;
+      }
+      q = make_uint4(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]), f2bf2(v[4], v[5]), f2bf2(v[6], v[7]));
+    }
+  }
+  __device__ __forceinline__ void store(unsigned char* row, int tid) const {
+    if (tid >= 2 * W) return;
+    const int p = tid >> 1, h = tid & 1;
+    *reinterpret_cast<uint2*>(row + rn_ioff(p, 2 * h)) = make_uint2(q.x, q.y);
+    *reinterpret_cast<uint2*>(row + rn_ioff(p, 2 * h + 1)) = make_uint2(q.z, q.w);
+  }
+};
+
+// Instruction order of a step: operand reads four ahead of their MFMAs (an
+// LDS read takes about as long as three pairs of MFMAs), and after each
+// operand's MFMAs a share of the activation arithmetic
+__device__ __forceinline__ void rn_interleave() {
+  __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);     // LDS reads
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);   // MFMAs
+    __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);   // VALU
+    if (i < 5) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+}
+
+template <int W, bool FIELDS>
+__global__ void __launch_bounds__(RowNet<W>::NT, 4) conv_rows_kernel(NetArgs a, int S, int strips) {
+  using P = RowNet<W>;
+  constexpr int HROW = P::HROW, IROW = P::IROW;
+  extern __shared__ __align__(16) unsigned char rnlds[];   // the input ring, then layers 0..3's
+  const int b = blockIdx.x / strips, y0 = (blockIdx.x - b * strips) * S;
+  const int rows = a.H - y0 < S ? a.H - y0 : S;
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave / P::WPG, part = wave % P::WPG;
+  int px[3];   // the lane's pixel of the fragment, shifted by -1, 0, 1
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const int c = part * 16 + m + d - 1;
+    px[d] = c < 0 ? c + W : (c >= W ? c - W : c);
+  }
+  int out[2];  // this group's ring (group 0: layer 0's)
+#pragma unroll
+  for (int j = 0; j < 2; ++j) out[j] = P::IB + group * P::HB + rn_off(px[1], 2 * j + (kq >> 1)) + (kq & 1) * 8;
+  const int steps = rows + 17;   // the last output row leaves a step after its MFMAs
+  if (group == 0) {
+    int off0[3], off4[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      off0[d] = rn_ioff(px[d], kq);
+      off4[d] = P::IB + 3 * P::HB + rn_off(px[d], kq);
+    }
+    // group 0 also brings the input: rows y0 - 5 .. y0 - 3 before the first
+    // step, then one a step, loaded a step ahead
+    RowInput<W, FIELDS> in;
+#pragma unroll 1
+    for (int r = 0; r < 3; ++r) {
+      in.load(a, b, y0 - 5 + r, tid);
+      in.store(rnlds + r * IROW, tid);
+    }
+    in.load(a, b, y0 - 2, tid);
+    RowWeights<16, 32> w0;
+    w0.load(a.w[0], a.bias[0], lane);
+    unsigned char* const wlast = rnlds + P::IB + 4 * P::HB;
+    for (int i = tid; i < 9 * 64; i += P::WPG * 64) {
+      const int t = i >> 6, l = i & 63;
+      *reinterpret_cast<uint4*>(wlast + i * 16) =
+          *reinterpret_cast<const uint4*>(a.w[4] + ((l & 15) * 9 + t) * 32 + (l >> 4) * 8);
+    }
+    const unsigned char* const wl = wlast + lane * 16;
+    float b4[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b4[i] = a.bias[4][4 * kq + i];
+    f32x4 accA[2], accB[2], oc;
+    accB[0] = accB[1] = oc = f32x4{0.f, 0.f, 0.f, 0.f};
+    lds_barrier();
+    auto step = [&](auto ph, int t, f32x4(&ac)[2], const f32x4(&ap)[2]) {
+      constexpr int PH = decltype(ph)::value;
+      in.store(rnlds + ((PH + 3) & 3) * IROW, tid);
+      in.load(a, b, y0 - 1 + t, tid);
+      const int r4 = y0 + t - 17;   // the output row of the step before
+      if (t >= 17 && t < rows + 17) {
+        const long gp = ((long)b * a.H + r4) * W + px[1];
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = oc[i] + b4[i];
+        if (!FIELDS) {
+          *reinterpret_cast<float4*>(&a.out[gp * 16 + 4 * kq]) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int co = 4 * kq + i;
+            if (co < a.cout) {
+              const float x = v[i] * a.out_scale[co];
+              a.dst[co][gp] = (double)x + (a.add[0] ? a.add[co][gp] : 0.0);
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      rn_conv<16, 32, IROW, PH>(rnlds, off0, w0, ac);
+      rn_hidden<16, HROW, PH + 3>(rnlds, out, w0, ap);
+      rn_interleave();
+      __builtin_amdgcn_sched_barrier(0);
+      rn_conv_last<HROW, PH>(rnlds, off4, wl, oc);
+      lds_barrier();
+    };
+    for (int t = 0;; t += 4) {
+      step(std::integral_constant<int, 0>{}, t, accA, accB);
+      if (t + 1 >= steps) break;
+      step(std::integral_constant<int, 1>{}, t + 1, accB, accA);
+      if (t + 2 >= steps) break;
+      step(std::integral_constant<int, 2>{}, t + 2, accA, accB);
+      if (t + 3 >= steps) break;
+      step(std::integral_constant<int, 3>{}, t + 3, accB, accA);
+      if (t + 4 >= steps) break;
+    }
+  } else {
+    int off[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) off[d] = P::IB + (group - 1) * P::HB + rn_off(px[d], kq);
+    RowWeights<32, 32> wt;
+    wt.load(a.w[group], a.bias[group], lane);
+    f32x4 accA[2], accB[2];
+    accB[0] = accB[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    lds_barrier();
+    auto step = [&](auto ph, f32x4(&ac)[2], const f32x4(&ap)[2]) {
+      constexpr int PH = decltype(ph)::value;
+      rn_conv<32, 32, HROW, PH>(rnlds, off, wt, ac);
+      rn_hidden<32, HROW, PH + 3>(rnlds, out, wt, ap);
+      rn_interleave();
+      lds_barrier();
+    };
+    for (int t = 0;; t += 4) {
+      step(std::integral_constant<int, 0>{}, accA, accB);
+      if (t + 1 >= steps) break;
+      step(std::integral_constant<int, 1>{}, accB, accA);
+      if (t + 2 >= steps) break;
+      step(std::integral_constant<int, 2>{}, accA, accB);
+      if (t + 3 >= steps) break;
+      step(std::integral_constant<int, 3>{}, accB, accA);
+      if (t + 4 >= steps) break;
+    }
+  }
+}
+
+template <int W, bool FIELDS>
+int launch_rows(const NetArgs& a, int S, hipStream_t s) {
+  using P = RowNet<W>;
+  constexpr int lds = P::lds_bytes();
+  static_assert(lds * P::WG_PER_CU <= 160 * 1024, "rings do not fit the LDS");
+  static bool attr = false;
+  if (!attr) {
+    const hipError_t e = hipFuncSetAttribute((const void*)conv_rows_kernel<W, FIELDS>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess)
+      return ddx::set_error(DDX_ERR_HIP, std::string("conv_rows LDS attribute: ") + hipGetErrorString(e));
+    attr = true;
+  }
+  const int strips = (a.H + S - 1) / S;
+  hipLaunchKernelGGL((conv_rows_kernel<W, FIELDS>), dim3((unsigned)(a.B * strips)), dim3(P::NT), lds, s, a, S, strips);
+  CL_LAUNCHCHK("conv_rows");
+  return 0;
+}
+
+// Strip height of the row kernel for B images of H rows, and the rounds of
+// steps it takes: the strips run in rounds of 256 CUs' workgroups, a strip of
+// S rows takes S + 17 steps.
+long rows_plan(int B, int H, int per_cu, int* S) {
+  long best = -1;
+  for (int n = 1; n <= 8 && n <= H; ++n) {
+    const int s = (H + n - 1) / n;
+    const long wgs = (long)B * ((H + s - 1) / s);
+    const long cost = ((wgs + 256L * per_cu - 1) / (256L * per_cu)) * (s + 17);
+    if (best < 0 || cost < best) { best = cost; *S = s; }
+  }
+  return best;
 }
 
 }  // namespace
@@ -1496,6 +1828,18 @@ int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
   const long big = (H % 16 == 0 && W % 32 == 0) ? (long)B * (H / 16) * (W / 32) : 0;
   const bool small_ok = H % 8 == 0 && W % 16 == 0;
   if (nl == 5 && hid == 32) {
+    // Row by row where its start and steps (6 us, then 1.4 us each with every
+    // CU busy) take less than the tile kernel's rounds of 256 tiles (26.5 us
+    // each): 256 images 64^2 112 us against 213, 128 images 72 against 107;
+    // for 64 images the two are even (53), below that the tiles win.
+    if (big >= 256 && (W == 32 || W == 64) && !x == !out) {
+      int S = 0;
+      const long steps = rows_plan(B, H, W == 64 ? RowNet<64>::WG_PER_CU : RowNet<32>::WG_PER_CU, &S);
+      if (60 + 14 * steps < 265 * ((big + 255) / 256)) {
+        if (W == 64) return x ? launch_rows<64, false>(a, S, s) : launch_rows<64, true>(a, S, s);
+        return x ? launch_rows<32, false>(a, S, s) : launch_rows<32, true>(a, S, s);
+      }
+    }
     if (big >= 256 || (big > 0 && !small_ok)) return launch_net<5, 32, 32, 16, 768>(a, s);
     // a few images: small tiles, whose layers are a few short dependent
     // phases each (one 64^2 image, a single coarse run: 4 x 4 tiles, one

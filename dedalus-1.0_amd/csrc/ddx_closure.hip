@@ -97,6 +97,8 @@ struct ConvArgs {
   float* out_f32;     // [npix][Co] or null
   uint16_t* out_bf16; // [npix][Co] or null
   int B, H, W, Ci, Co, mode;
+  int cout;           // channels per pixel of out_f32 (Co, or fewer: only those are stored)
+  double* bpart;      // GELU_GRAD, tile kernel: [gridDim.x][Co] sums of the fp32 result over a block's pixels, or null
 };
 
 // One wavefront: 16 consecutive pixels x all Co = 16*NCO output channels.
@@ -147,7 +149,7 @@ __global__ void __launch_bounds__(256) conv3x3_kernel(ConvArgs a) {
         v += bv;
         act = a.mode == DDX_CONV_GELU ? gelu(v) : v;
       }
-      if (a.out_f32) a.out_f32[o] = v;
+      if (a.out_f32 && c < a.cout) a.out_f32[(p0 + 4 * kq + i) * a.cout + c] = v;
       if (a.out_bf16) a.out_bf16[o] = f2bf(act);
     }
   }
@@ -167,6 +169,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
+// eight consecutive bf16 from LDS (16-byte aligned)
+__device__ inline bf16x8 lds16(const uint16_t* p) {
+  const uint4 v = *reinterpret_cast<const uint4*>(p);
+  const u32x4 u = {v.x, v.y, v.z, v.w};
+  return __builtin_bit_cast(bf16x8, u);
+}
+
 // eight consecutive bf16 from LDS as two 8-byte reads
 __device__ inline bf16x8 lds8(const uint16_t* p) {
   const uint2 lo = *reinterpret_cast<const uint2*>(p);
@@ -175,12 +184,16 @@ __device__ inline bf16x8 lds8(const uint16_t* p) {
   return __builtin_bit_cast(bf16x8, v);
 }
 
-// LDS-tiled 3x3 convolution for CI, CO in {16, 32}, W % 64 == 0, H % 4 == 0.
-// Output tile = 4 rows x 64 columns of one image; wavefront w owns row
-// y0 + w as four 16-pixel fragments.  Blocks loop over tiles (tile c,
+// LDS-tiled 3x3 convolution for CI, CO in {16, 32}.  Output tile = 256 pixels
+// of one image, 4 rows x 64 columns (TC = 64) or 8 x 32 (TC = 32); wavefront w
+// owns 64 of them as four 16-pixel fragments.  Blocks loop over tiles (tile c,
 // c + gridDim.x, ...): the weights are staged in LDS once per block, and the
-// next tile's 6 x 66 input halo is loaded into registers while the current
-// tile computes.  Pixel stride and weight-row stride CI + 4 (bf16) place the
+// next tile's input halo is loaded into registers while the current tile
+// computes.  The first halo and, for the GELU gradient, a tile's
+// pre-activations are requested before anything waits: with one tile per
+// block (a training batch of 32 images 64^2) the kernel is a chain of memory
+// latencies.  TC = 32 multiplies 32 channels in two steps of 16, the sums of
+// conv3x3_kernel.  Pixel stride and weight-row stride CI + 4 (bf16) place the
 // 16 rows of a fragment read in distinct bank pairs.  CI = 32 uses the
 // gfx950 16x16x32 bf16 MFMA, CI = 16 the 16x16x16 one.
 //
@@ -188,10 +201,10 @@ __device__ inline bf16x8 lds8(const uint16_t* p) {
 // pass): bias and activation are applied to the accumulators and the
 // results staged as bf16, which halves the staging LDS; the kernel then fits
 // three workgroups per CU instead of two.
-template <int CI, int CO, bool BF>
-__global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntiles) {
+template <int CI, int CO, bool BF, int TC>
+__global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs a, long ntiles) {
   constexpr int PS = CI + 4, WS = CI + 4;
-  constexpr int HR = 6, HC = 66;
+  constexpr int TR = 256 / TC, HR = TR + 2, HC = TC + 2;
   constexpr int NCO = CO / 16;
   constexpr int CK = CI / 8;                       // 16-byte chunks per pixel
   constexpr int NH = HR * HC * CK, HPT = (NH + 255) / 256;
@@ -205,25 +218,7 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
   __shared__ __align__(16) uint16_t halo[BUF_B / 2];
   __shared__ __align__(16) uint16_t wl[CO * 9 * WS];
   const int tid = threadIdx.x;
-  const int tiles_x = a.W / 64, tiles_y = a.H / 4;
-  {
-    uint4 wv[WPT];
-#pragma unroll
-    for (int k = 0; k < WPT; ++k) {
-      const int i = tid + k * 256;
-      if (i < NW) wv[k] = *reinterpret_cast<const uint4*>(&a.w[(long)i * 8]);
-    }
-#pragma unroll
-    for (int k = 0; k < WPT; ++k) {
-      const int i = tid + k * 256;
-      if (i < NW) {
-        const int row = i / CK, ch = i - row * CK;
-        uint2* d = reinterpret_cast<uint2*>(&wl[row * WS + ch * 8]);
-        d[0] = make_uint2(wv[k].x, wv[k].y);
-        d[1] = make_uint2(wv[k].z, wv[k].w);
-      }
-    }
-  }
+  const int tiles_x = a.W / TC, tiles_y = a.H / TR;
   uint4 hv[HPT];
   auto fetch = [&](long tile) {
     long rest = tile;
@@ -231,7 +226,7 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
     rest /= tiles_x;
     const int ty = (int)(rest % tiles_y);
     const int b = (int)(rest / tiles_y);
-    const int x0 = tx * 64, y0 = ty * 4;
+    const int x0 = tx * TC, y0 = ty * TR;
 #pragma unroll
     for (int k = 0; k < HPT; ++k) {
       const int i = tid + k * 256;
@@ -259,6 +254,26 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
   }
   long tile = blockIdx.x;
   if (tile < ntiles) fetch(tile);
+  uint4 wv[WPT];
+#pragma unroll
+  for (int k = 0; k < WPT; ++k) {
+    const int i = tid + k * 256;
+    if (i < NW) wv[k] = *reinterpret_cast<const uint4*>(&a.w[(long)i * 8]);
+  }
+#pragma unroll
+  for (int k = 0; k < WPT; ++k) {
+    const int i = tid + k * 256;
+    if (i < NW) {
+      const int row = i / CK, ch = i - row * CK;
+      uint2* d = reinterpret_cast<uint2*>(&wl[row * WS + ch * 8]);
+      d[0] = make_uint2(wv[k].x, wv[k].y);
+      d[1] = make_uint2(wv[k].z, wv[k].w);
+    }
+  }
+  double bsum[4] = {0.0, 0.0, 0.0, 0.0};   // this thread's channels (lane % (CO/4)) * 4 + e over its pixels
+  // pixel px of the wavefront's 64: tile row and column
+  auto prow = [&](int px) { return TC == 64 ? wave : 2 * wave + (px >> 5); };
+  auto pcol = [&](int px) { return TC == 64 ? px : px & 31; };
   for (; tile < ntiles; tile += gridDim.x) {
     lds_barrier();  // the previous tile's fragment reads are done
 #pragma unroll
@@ -274,6 +289,23 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
     lds_barrier();
     const long next = tile + gridDim.x;
     if (next < ntiles) fetch(next);  // in flight while this tile computes
+    long rest = tile;
+    const int tx = (int)(rest % tiles_x);
+    rest /= tiles_x;
+    const int ty = (int)(rest % tiles_y);
+    const int b = (int)(rest / tiles_y);
+    // first pixel of the tile row r
+    const long p00 = ((long)b * a.H + ty * TR) * a.W + tx * TC;
+    auto gpix = [&](int px) { return p00 + (long)prow(px) * a.W + pcol(px); };
+    // pre-activations of this thread's output chunks (see the staging below)
+    constexpr int C4 = CO / 4, NR = C4;
+    const int c = (lane % C4) * 4;
+    float4 zaux[NR];
+    if (!BF && grad) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+        zaux[r] = *reinterpret_cast<const float4*>(&a.aux[gpix((lane + 64 * r) / C4) * CO + c]);
+    }
     f32x4 acc[4][NCO];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -282,7 +314,7 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
       const int dy = t / 3, dx = t % 3;
-      if constexpr (CI % 32 == 0) {
+      if constexpr (CI % 32 == 0 && TC == 64) {
 #pragma unroll
         for (int kc = 0; kc < CI / 32; ++kc) {
           bf16x8 bv[NCO];
@@ -290,7 +322,7 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
           for (int j = 0; j < NCO; ++j) bv[j] = lds8(&wl[((j * 16 + m) * 9 + t) * WS + kc * 32 + 8 * kq]);
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const bf16x8 av = lds8(&halo[((wave + dy) * HC + q * 16 + m + dx) * PS + kc * 32 + 8 * kq]);
+            const bf16x8 av = lds8(&halo[((prow(q * 16) + dy) * HC + pcol(q * 16) + m + dx) * PS + kc * 32 + 8 * kq]);
 #pragma unroll
             for (int j = 0; j < NCO; ++j)
               acc[q][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[j], acc[q][j], 0, 0, 0);
@@ -304,7 +336,7 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
           for (int j = 0; j < NCO; ++j) bv[j] = lds4(&wl[((j * 16 + m) * 9 + t) * WS + kc * 16 + 4 * kq]);
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const bf16x4 av = lds4(&halo[((wave + dy) * HC + q * 16 + m + dx) * PS + kc * 16 + 4 * kq]);
+            const bf16x4 av = lds4(&halo[((prow(q * 16) + dy) * HC + pcol(q * 16) + m + dx) * PS + kc * 16 + 4 * kq]);
 #pragma unroll
             for (int j = 0; j < NCO; ++j)
               acc[q][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv[j], acc[q][j], 0, 0, 0);
@@ -312,12 +344,6 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
         }
       }
     }
-    long rest = tile;
-    const int tx = (int)(rest % tiles_x);
-    rest /= tiles_x;
-    const int ty = (int)(rest % tiles_y);
-    const int b = (int)(rest / tiles_y);
-    const long prow = ((long)b * a.H + ty * 4 + wave) * a.W + tx * 64;
     lds_barrier();  // every wavefront is done with the halo
     if constexpr (BF) {
       // activations of the D fragments (pixel q*16 + 4kq + i, channel j*16 + m)
@@ -333,12 +359,10 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
             sb[(q * 16 + 4 * kq + i) * EB + j * 16 + m] = f2bf(gelu_on ? gelu(v) : v);
           }
       lds_barrier();
-      constexpr int C4 = CO / 4, NR = (64 * C4) / 64;
-      const int c = (lane % C4) * 4;
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         const int px = (lane + 64 * r) / C4;
-        *reinterpret_cast<uint2*>(&a.out_bf16[(prow + px) * CO + c]) =
+        *reinterpret_cast<uint2*>(&a.out_bf16[gpix(px) * CO + c]) =
             *reinterpret_cast<const uint2*>(&sb[px * EB + c]);
       }
       continue;
@@ -352,32 +376,21 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
 #pragma unroll
         for (int i = 0; i < 4; ++i) st[(q * 16 + 4 * kq + i) * ES + j * 16 + m] = acc[q][j][i];
     lds_barrier();
-    // the wavefront's 64 pixels x CO channels are contiguous in HBM: 4 channels
-    // per chunk; a lane's channels c..c+3 are the same in every chunk (C4
-    // divides 64), so its bias was read once before the tile loop.  The aux
-    // loads of all chunks are issued before any is used.
-    constexpr int C4 = CO / 4, NR = (64 * C4) / 64;
-    const int c = (lane % C4) * 4;
-    float4 zaux[NR];
-    if (grad) {
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        const int px = (lane + 64 * r) / C4;
-        zaux[r] = *reinterpret_cast<const float4*>(&a.aux[(prow + px) * CO + c]);
-      }
-    }
+    // 4 channels per chunk; a lane's channels c..c+3 are the same in every
+    // chunk (C4 divides 64), so its bias was read once before the tile loop
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       const int px = (lane + 64 * r) / C4;
       const float4 d = *reinterpret_cast<const float4*>(&st[px * ES + c]);
       float v[4] = {d.x, d.y, d.z, d.w}, act[4];
-      const long o = (prow + px) * CO + c;
+      const long gp = gpix(px), o = gp * CO + c;
       if (grad) {
         const float zz[4] = {zaux[r].x, zaux[r].y, zaux[r].z, zaux[r].w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           v[e] *= gelu_grad(zz[e]);
           act[e] = v[e];
+          bsum[e] += (double)v[e];
         }
       } else {
 #pragma unroll
@@ -386,11 +399,35 @@ __global__ void __launch_bounds__(256) conv3x3_tile_kernel(ConvArgs a, long ntil
           act[e] = gelu_on ? gelu(v[e]) : v[e];
         }
       }
-      if (a.out_f32) *reinterpret_cast<float4*>(&a.out_f32[o]) = make_float4(v[0], v[1], v[2], v[3]);
+      if (a.out_f32) {
+        if (a.cout == CO) {
+          *reinterpret_cast<float4*>(&a.out_f32[o]) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (c + e < a.cout) a.out_f32[gp * a.cout + c + e] = v[e];
+        }
+      }
       if (a.out_bf16)
         *reinterpret_cast<uint2*>(&a.out_bf16[o]) =
             make_uint2((uint32_t)f2bf(act[0]) | ((uint32_t)f2bf(act[1]) << 16),
                        (uint32_t)f2bf(act[2]) | ((uint32_t)f2bf(act[3]) << 16));
+    }
+  }
+  if constexpr (!BF) {
+    if (a.bpart) {
+      // lanes, then wavefronts, in a fixed order
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int d = CO / 4; d < 64; d *= 2) bsum[e] += __shfl_xor(bsum[e], d);
+      lds_barrier();
+      double* sh = reinterpret_cast<double*>(halo);
+      if (lane < CO / 4)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sh[wave * CO + lane * 4 + e] = bsum[e];
+      lds_barrier();
+      if (tid < CO) a.bpart[(long)blockIdx.x * CO + tid] = ((sh[tid] + sh[CO + tid]) + sh[2 * CO + tid]) + sh[3 * CO + tid];
     }
   }
 }
@@ -446,37 +483,46 @@ __global__ void __launch_bounds__(64) conv3x3_wgrad_kernel(const uint16_t* __res
     }
 }
 
-// LDS-tiled weight gradient for CI, CO in {16, 32}, W % 64 == 0, H % 4 == 0.
-// Block c accumulates over output tiles c, c + gridDim.x, ... (tile = 4 rows
-// x 64 columns of one image, as in the forward kernel) and writes
+// LDS-tiled weight gradient for CI, CO in {16, 32}.  Block c accumulates over
+// output tiles c, c + gridDim.x, ... (256 pixels of one image, 4 x 64 for TC =
+// 64 and 8 x 32 for TC = 32, as in the forward kernel) and writes
 // partial[c][co][t][ci].  Per tile, dz (256 pixels x CO) and the input halo
-// (6 x 66 pixels x CI) are staged channel-major, so the MFMA's K dimension
-// (pixels) is contiguous: A[m = co][k = p] from dzT[co][p] (8-byte reads),
-// B[k = p][n = ci] from haloT[ci][row][col].  Wavefront w owns the
-// (co tile, ci tile) pairs w, w + 4, ... with all nine tap accumulators.
+// are staged channel-major, so the MFMA's K dimension (32 pixels) is
+// contiguous: A[m = co][k = p] from dzT[co][p] (16-byte reads), B[k = p][n =
+// ci] from haloT[ci][row][col].  The three column shifts of a row come from
+// one run of five 4-byte words, shifted in registers by 16 bits for the odd
+// one; reading each shifted operand as eight 2-byte words took 36 LDS
+// instructions per 16 pixels where this takes 15 per 32 (18.6 -> 11 us for 32
+// channels and 32 images 64^2).  The transposed staging writes pixel pairs.
+// Wavefront w owns the (co tile, ci tile) pairs w, w + 4, ... with all nine
+// tap accumulators.  The next tile's loads are in flight while one computes.
 //
 // With dzf (the fp32 dz), the block also sums dz over its pixels per output
 // channel in double (the bias gradient), thread t taking channel t mod CO and
 // every (256 / CO)-th pixel, combined in a fixed order into
 // bpartial[block][co]: the column sums ride along with the tiles this
 // kernel reads anyway, instead of a separate pass over dz.
-template <int CI, int CO>
+template <int CI, int CO, int TC>
 __global__ void __launch_bounds__(256) conv3x3_wgrad_tile_kernel(const uint16_t* __restrict__ x,
                                                                  const uint16_t* __restrict__ dz,
                                                                  float* __restrict__ partial,
                                                                  int B, int H, int W,
                                                                  const float* __restrict__ dzf = nullptr,
                                                                  double* __restrict__ bpartial = nullptr) {
-  constexpr int DS = 260;            // dzT row stride (bf16): 256 pixels + 4
-  constexpr int HRS = 68;            // halo row stride (66 columns + 2)
-  constexpr int HS = 6 * HRS + 2;    // halo channel stride, odd in 4-byte words
+  constexpr int TR = 256 / TC, HR = TR + 2, HC = TC + 2;
+  constexpr int DS = 264;            // dzT row stride (bf16): 16-byte rows, 16 rows on distinct banks
+  constexpr int HRS = TC + 4;        // halo row stride
+  constexpr int HS = HR * HRS + 2;   // halo channel stride, odd in 4-byte words
+  static_assert((HS / 2) % 2 == 1 && HS % 2 == 0, "halo channel stride");
   constexpr int NCT = CI / 16, NPAIR = (CO / 16) * (CI / 16);
   constexpr int NPW = (NPAIR + 3) / 4;  // pairs per wavefront
+  constexpr int ND = 128 * (CO / 4), DPT = (ND + 255) / 256;            // dz pixel pairs x 4 channels
+  constexpr int NH = HR * (HC / 2) * (CI / 4), HPT = (NH + 255) / 256;  // halo pixel pairs x 4 channels
   __shared__ __align__(16) uint16_t dzT[CO * DS];
   __shared__ __align__(16) uint16_t haloT[CI * HS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int m = lane & 15, kq = lane >> 4;
-  const int tiles_x = W / 64, tiles_y = H / 4;
+  const int tiles_x = W / TC, tiles_y = H / TR;
   const long ntiles = (long)B * tiles_y * tiles_x;
   f32x4 acc[NPW][9];
 #pragma unroll
@@ -486,68 +532,98 @@ __global__ void __launch_bounds__(256) conv3x3_wgrad_tile_kernel(const uint16_t*
   constexpr int PG = 256 / CO;              // pixel groups of the bias sums
   const int bco = tid % CO, bpg = tid / CO;
   double bsum = 0.0;
-  for (long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+  uint2 dv[DPT][2], hv[HPT][2];
+  float bv[256 / PG];
+  auto fetch = [&](long tile) {
     long rest = tile;
     const int tx = (int)(rest % tiles_x);
     rest /= tiles_x;
     const int ty = (int)(rest % tiles_y);
     const int b = (int)(rest / tiles_y);
-    const int x0 = tx * 64, y0 = ty * 4;
+    const int x0 = tx * TC, y0 = ty * TR;
+#pragma unroll
+    for (int k = 0; k < DPT; ++k) {
+      const int i = tid + k * 256;
+      if (i < ND) {
+        const int pp = i / (CO / 4), ch = (i - pp * (CO / 4)) * 4, pix = 2 * pp;
+        const uint16_t* q = &dz[(((long)b * H + y0 + pix / TC) * W + x0 + pix % TC) * CO + ch];
+        dv[k][0] = *reinterpret_cast<const uint2*>(q);
+        dv[k][1] = *reinterpret_cast<const uint2*>(q + CO);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < HPT; ++k) {
+      const int i = tid + k * 256;
+      if (i < NH) {
+        const int pp = i / (CI / 4), ch = (i - pp * (CI / 4)) * 4;
+        const int r = pp / (HC / 2), c = 2 * (pp - r * (HC / 2));
+        const long row = ((long)b * H + wrapi(y0 - 1 + r, H)) * W;
+        hv[k][0] = *reinterpret_cast<const uint2*>(&x[(row + wrapi(x0 - 1 + c, W)) * CI + ch]);
+        hv[k][1] = *reinterpret_cast<const uint2*>(&x[(row + wrapi(x0 + c, W)) * CI + ch]);
+      }
+    }
     if (dzf) {
-      // loads first, then the double adds in pixel order
-      float bv[256 / PG];
 #pragma unroll
       for (int k = 0; k < 256 / PG; ++k) {
         const int pix = bpg + PG * k;
-        bv[k] = dzf[(((long)b * H + y0 + (pix >> 6)) * W + x0 + (pix & 63)) * CO + bco];
+        bv[k] = dzf[(((long)b * H + y0 + pix / TC) * W + x0 + pix % TC) * CO + bco];
       }
-#pragma unroll
-      for (int k = 0; k < 256 / PG; ++k) bsum += (double)bv[k];
     }
+  };
+  // four channels of two adjacent pixels -> one 4-byte word per channel
+  auto put = [](uint16_t* base, int stride, int o, const uint2 (&v)[2]) {
+    *reinterpret_cast<uint32_t*>(&base[o]) = __builtin_amdgcn_perm(v[1].x, v[0].x, 0x05040100u);
+    *reinterpret_cast<uint32_t*>(&base[o + stride]) = __builtin_amdgcn_perm(v[1].x, v[0].x, 0x07060302u);
+    *reinterpret_cast<uint32_t*>(&base[o + 2 * stride]) = __builtin_amdgcn_perm(v[1].y, v[0].y, 0x05040100u);
+    *reinterpret_cast<uint32_t*>(&base[o + 3 * stride]) = __builtin_amdgcn_perm(v[1].y, v[0].y, 0x07060302u);
+  };
+  long tile = blockIdx.x;
+  if (tile < ntiles) fetch(tile);
+  for (; tile < ntiles; tile += gridDim.x) {
     lds_barrier();  // the previous tile's reads are done
-    // dz: 256 pixels x CO, 4 channels per load, stored transposed
-    for (int i = tid; i < 256 * (CO / 4); i += 256) {
-      const int pix = i / (CO / 4), ch = (i - pix * (CO / 4)) * 4;
-      const int r = pix >> 6, c = pix & 63;
-      const uint2 v = *reinterpret_cast<const uint2*>(
-          &dz[(((long)b * H + y0 + r) * W + x0 + c) * CO + ch]);
-      dzT[(ch + 0) * DS + pix] = (uint16_t)(v.x & 0xffffu);
-      dzT[(ch + 1) * DS + pix] = (uint16_t)(v.x >> 16);
-      dzT[(ch + 2) * DS + pix] = (uint16_t)(v.y & 0xffffu);
-      dzT[(ch + 3) * DS + pix] = (uint16_t)(v.y >> 16);
+#pragma unroll
+    for (int k = 0; k < DPT; ++k) {
+      const int i = tid + k * 256;
+      if (i < ND) {
+        const int pp = i / (CO / 4), ch = (i - pp * (CO / 4)) * 4;
+        put(dzT, DS, ch * DS + 2 * pp, dv[k]);
+      }
     }
-    // halo: 6 x 66 pixels x CI, stored transposed
-    for (int i = tid; i < 6 * 66 * (CI / 4); i += 256) {
-      const int pix = i / (CI / 4), ch = (i - pix * (CI / 4)) * 4;
-      const int r = pix / 66, c = pix - r * 66;
-      const int yy = wrapi(y0 - 1 + r, H), xx = wrapi(x0 - 1 + c, W);
-      const uint2 v = *reinterpret_cast<const uint2*>(
-          &x[(((long)b * H + yy) * W + xx) * CI + ch]);
-      const int o = r * HRS + c;
-      haloT[(ch + 0) * HS + o] = (uint16_t)(v.x & 0xffffu);
-      haloT[(ch + 1) * HS + o] = (uint16_t)(v.x >> 16);
-      haloT[(ch + 2) * HS + o] = (uint16_t)(v.y & 0xffffu);
-      haloT[(ch + 3) * HS + o] = (uint16_t)(v.y >> 16);
+#pragma unroll
+    for (int k = 0; k < HPT; ++k) {
+      const int i = tid + k * 256;
+      if (i < NH) {
+        const int pp = i / (CI / 4), ch = (i - pp * (CI / 4)) * 4;
+        const int r = pp / (HC / 2), c = 2 * (pp - r * (HC / 2));
+        put(haloT, HS, ch * HS + r * HRS + c, hv[k]);
+      }
+    }
+    if (dzf) {
+#pragma unroll
+      for (int k = 0; k < 256 / PG; ++k) bsum += (double)bv[k];   // in pixel order
     }
     lds_barrier();
+    if (tile + gridDim.x < ntiles) fetch(tile + gridDim.x);
 #pragma unroll
     for (int u = 0; u < NPW; ++u) {
       const int pair = wave + 4 * u;
       if (pair >= NPAIR) break;
       const int co0 = (pair / NCT) * 16, ci0 = (pair % NCT) * 16;
-      for (int ks = 0; ks < 16; ++ks) {       // 16 pixels per K step
-        const int row = ks >> 2, col0 = (ks & 3) * 16;
-        const bf16x4 av = lds4(&dzT[(co0 + m) * DS + ks * 16 + 4 * kq]);
-        const uint16_t* hb = &haloT[(ci0 + m) * HS];
+      const uint16_t* hb = &haloT[(ci0 + m) * HS + 8 * kq];
+#pragma unroll 2
+      for (int ks = 0; ks < 8; ++ks) {       // 32 pixels per K step
+        const int row = (ks * 32) / TC, col0 = (ks * 32) % TC;
+        const bf16x8 av = lds16(&dzT[(co0 + m) * DS + ks * 32 + 8 * kq]);
 #pragma unroll
-        for (int t = 0; t < 9; ++t) {
-          const uint16_t* hp = hb + (row + t / 3) * HRS + col0 + 4 * kq + t % 3;
-          bf16x4 bv;
-          bv[0] = (short)hp[0];
-          bv[1] = (short)hp[1];
-          bv[2] = (short)hp[2];
-          bv[3] = (short)hp[3];
-          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[u][t], 0, 0, 0);
+        for (int dy = 0; dy < 3; ++dy) {
+          const uint32_t* hp = reinterpret_cast<const uint32_t*>(hb + (row + dy) * HRS + col0);
+          const uint32_t d0 = hp[0], d1 = hp[1], d2 = hp[2], d3 = hp[3], d4 = hp[4];
+          const u32x4 s0 = {d0, d1, d2, d3}, s2 = {d1, d2, d3, d4};
+          const u32x4 s1 = {__builtin_amdgcn_alignbit(d1, d0, 16), __builtin_amdgcn_alignbit(d2, d1, 16),
+                            __builtin_amdgcn_alignbit(d3, d2, 16), __builtin_amdgcn_alignbit(d4, d3, 16)};
+          acc[u][3 * dy] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, s0), acc[u][3 * dy], 0, 0, 0);
+          acc[u][3 * dy + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, s1), acc[u][3 * dy + 1], 0, 0, 0);
+          acc[u][3 * dy + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, s2), acc[u][3 * dy + 2], 0, 0, 0);
         }
       }
     }
@@ -580,10 +656,26 @@ __global__ void __launch_bounds__(256) conv3x3_wgrad_tile_kernel(const uint16_t*
 
 // out[j] = sum over chunks of partial[c][j] in a fixed order (double):
 // block = 64 consecutive j x SUM_GROUPS chunk groups (group q sums chunks q,
-// q + SUM_GROUPS, ... with four loads in flight), the group sums are then
+// q + SUM_GROUPS, ... with eight loads in flight), the group sums are then
 // added in group order.  Sixteen groups keep ~150 k threads loading (a
 // 32 x 32 layer's 9216 weights x 512 chunks is 19 MB).
 constexpr int SUM_GROUPS = 16;
+
+// chunks q, q + SUM_GROUPS, ... of one element, loads of eight chunks in flight
+template <typename T>
+__device__ inline double chunk_sum(const T* p, long stride, int nchunk, int q) {
+  double s = 0.0;
+  int c = q;
+  for (; c + 7 * SUM_GROUPS < nchunk; c += 8 * SUM_GROUPS) {
+    T v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = p[(long)(c + k * SUM_GROUPS) * stride];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k];
+  }
+  for (; c < nchunk; c += SUM_GROUPS) s += p[(long)c * stride];
+  return s;
+}
 
 __global__ void __launch_bounds__(64 * SUM_GROUPS) sum_chunks_kernel(const float* __restrict__ partial,
                                                                      float* __restrict__ out,
@@ -592,20 +684,7 @@ __global__ void __launch_bounds__(64 * SUM_GROUPS) sum_chunks_kernel(const float
   const int e = threadIdx.x & 63, q = threadIdx.x >> 6;
   const long j = (long)blockIdx.x * 64 + e;
   const long jc = j < n ? j : n - 1;   // in-range address for the spare lanes
-  double s = 0.0;
-  int c = q;
-  for (; c + 3 * SUM_GROUPS < nchunk; c += 4 * SUM_GROUPS) {
-    const float v0 = partial[(long)c * n + jc];
-    const float v1 = partial[(long)(c + SUM_GROUPS) * n + jc];
-    const float v2 = partial[(long)(c + 2 * SUM_GROUPS) * n + jc];
-    const float v3 = partial[(long)(c + 3 * SUM_GROUPS) * n + jc];
-    s += v0;
-    s += v1;
-    s += v2;
-    s += v3;
-  }
-  for (; c < nchunk; c += SUM_GROUPS) s += partial[(long)c * n + jc];
-  sh[q][e] = s;
+  sh[q][e] = chunk_sum(partial + jc, n, nchunk, q);
   __syncthreads();
   if (q == 0 && j < n) {
     double t = sh[0][e];
@@ -857,6 +936,316 @@ int check_conv(int B, int H, int W, int Ci, int Co) {
 
 inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
+// Tile width of the LDS-tiled kernels: 64 or 32 columns, 0 where they do not
+// apply
+int tile_cols(int H, int W, int Ci, int Co) {
+  if ((Ci != 16 && Ci != 32) || (Co != 16 && Co != 32)) return 0;
+  if (W % 64 == 0 && H % 4 == 0) return 64;
+  if (W % 32 == 0 && H % 8 == 0) return 32;
+  return 0;
+}
+
+// blocks loop over tiles; about four resident blocks per CU cover the chip
+inline long conv_blocks(long ntiles) { return ntiles < 1024 ? ntiles : 1024; }
+
+template <int CI, int CO, bool BF>
+void conv_tile_go(hipStream_t s, const ConvArgs& a, int tc) {
+  const long ntiles = (long)a.B * a.H * a.W / 256;
+  const dim3 grid((unsigned)conv_blocks(ntiles));
+  if (tc == 64) hipLaunchKernelGGL((conv3x3_tile_kernel<CI, CO, BF, 64>), grid, dim3(256), 0, s, a, ntiles);
+  else hipLaunchKernelGGL((conv3x3_tile_kernel<CI, CO, BF, 32>), grid, dim3(256), 0, s, a, ntiles);
+}
+
+template <bool BF>
+void conv_tile(hipStream_t s, const ConvArgs& a, int tc) {
+  switch (a.Ci * 100 + a.Co) {
+    case 1616: conv_tile_go<16, 16, BF>(s, a, tc); break;
+    case 1632: conv_tile_go<16, 32, BF>(s, a, tc); break;
+    case 3216: conv_tile_go<32, 16, BF>(s, a, tc); break;
+    default: conv_tile_go<32, 32, BF>(s, a, tc); break;
+  }
+}
+
+// ddx_conv3x3 with out_f32 holding cout <= Co channels per pixel
+int conv_run(hipStream_t s, int B, int H, int W, int Ci, int Co, const void* x, const void* w, const float* bias,
+             const float* aux, int mode, float* out_f32, void* out_bf16, int cout) {
+  int rc = check_conv(B, H, W, Ci, Co);
+  if (rc) return rc;
+  if (!x || !w || (!out_f32 && !out_bf16)) return ddx::set_error(DDX_ERR_ARG, "null argument");
+  if (mode != DDX_CONV_LINEAR && mode != DDX_CONV_GELU && mode != DDX_CONV_GELU_GRAD)
+    return ddx::set_error(DDX_ERR_ARG, "unknown convolution mode");
+  if (mode == DDX_CONV_GELU_GRAD && !aux)
+    return ddx::set_error(DDX_ERR_ARG, "DDX_CONV_GELU_GRAD needs the pre-activation");
+  ConvArgs a{(const uint16_t*)x, (const uint16_t*)w, bias, aux, out_f32, (uint16_t*)out_bf16,
+             B, H, W, Ci, Co, mode, cout, nullptr};
+  auto al = [](const void* q, uintptr_t n) { return ((uintptr_t)q % n) == 0; };
+  const bool aligned = al(x, 16) && al(w, 16) && al(out_f32, 16) && al(aux, 16) && al(out_bf16, 8);
+  const int tc = aligned ? tile_cols(H, W, Ci, Co) : 0;
+  if (tc) {
+    // bf16-only output without the GELU gradient stages bf16 (BF)
+    if (!out_f32 && mode != DDX_CONV_GELU_GRAD) conv_tile<true>(s, a, tc);
+    else conv_tile<false>(s, a, tc);
+    CL_LAUNCHCHK("conv3x3 tile");
+    return 0;
+  }
+  const long tiles = (long)B * H * W / 16;
+  const dim3 grid(nblk(tiles, 4));
+  switch (Co / 16) {
+    case 1: hipLaunchKernelGGL(conv3x3_kernel<1>, grid, dim3(256), 0, s, a); break;
+    case 2: hipLaunchKernelGGL(conv3x3_kernel<2>, grid, dim3(256), 0, s, a); break;
+    case 3: hipLaunchKernelGGL(conv3x3_kernel<3>, grid, dim3(256), 0, s, a); break;
+    default: hipLaunchKernelGGL(conv3x3_kernel<4>, grid, dim3(256), 0, s, a); break;
+  }
+  CL_LAUNCHCHK("conv3x3");
+  return 0;
+}
+
+template <int CI, int CO>
+void wgrad_go(hipStream_t s, int nch, int tc, const uint16_t* x, const uint16_t* dz, const float* dzf, float* partial,
+              double* bpartial, int B, int H, int W) {
+  if (tc == 64)
+    hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<CI, CO, 64>), dim3(nch), dim3(256), 0, s, x, dz, partial, B, H, W,
+                       dzf, bpartial);
+  else
+    hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<CI, CO, 32>), dim3(nch), dim3(256), 0, s, x, dz, partial, B, H, W,
+                       dzf, bpartial);
+}
+
+// The tile kernel's partial sums (tc columns per tile); returns their number
+int wgrad_tiles(hipStream_t s, int B, int H, int W, int Ci, int Co, int tc, const void* x, const void* dz,
+                const float* dzf, float* partial, double* bpartial, int nchunk) {
+  const long ntiles = (long)B * H * W / 256;
+  const int nch = (int)(ntiles < nchunk ? ntiles : nchunk);
+  const uint16_t* xx = (const uint16_t*)x;
+  const uint16_t* dd = (const uint16_t*)dz;
+  switch (Ci * 100 + Co) {
+    case 1616: wgrad_go<16, 16>(s, nch, tc, xx, dd, dzf, partial, bpartial, B, H, W); break;
+    case 1632: wgrad_go<16, 32>(s, nch, tc, xx, dd, dzf, partial, bpartial, B, H, W); break;
+    case 3216: wgrad_go<32, 16>(s, nch, tc, xx, dd, dzf, partial, bpartial, B, H, W); break;
+    default: wgrad_go<32, 32>(s, nch, tc, xx, dd, dzf, partial, bpartial, B, H, W); break;
+  }
+  return nch;
+}
+
+// ---------------------------------------------------------------------------
+// Training: the forward pass that keeps what the backward pass needs, and the
+// backward pass, as two native calls.  Issued layer by layer from Python, a
+// step of a five-layer network was 45 launches and as many allocations, 780 us
+// of host time around 300 us of kernels for 32 images 64^2; 6 launches forward
+// and 11 backward take 370 us, of which the loss and autograd's own work are
+// about half.
+// ---------------------------------------------------------------------------
+constexpr int TRAIN_L = 8;   // layers per preparing or summing launch; deeper networks take several
+
+inline int pad16(int c) { return (c + 15) / 16 * 16; }
+
+struct PrepLayer {
+  const float* w;   // (co, ci, ky, kx)
+  const float* b;
+  uint16_t* wf;     // as wprep_kernel
+  uint16_t* wt;
+  float* bp;        // bias padded with zeros to cop
+  int co, ci, cop, cip;
+  int end;          // elements of the layers up to this one
+};
+
+struct PrepArgs {
+  PrepLayer l[TRAIN_L];
+  int nl, nw;       // nw = l[nl - 1].end
+  const float* x;   // [npix][C]
+  uint16_t* xb;     // [npix][16]
+  long npix;        // 0: no input in this launch
+  int C;
+};
+
+// bf16 of 8 of a pixel's 16 padded channels
+__device__ inline uint4 pack8(const float (&v)[8]) {
+  uint32_t h[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) h[k] = (uint32_t)f2bf(v[2 * k]) | ((uint32_t)f2bf(v[2 * k + 1]) << 16);
+  return make_uint4(h[0], h[1], h[2], h[3]);
+}
+
+// All layers' weights and biases, and the input rounded to bf16: one thread
+// per padded weight, then one per 8 channels (16 bytes) of a pixel
+__global__ void __launch_bounds__(256) net_prep_kernel(PrepArgs a) {
+  const long j = (long)blockIdx.x * 256 + threadIdx.x;
+  if (j < a.nw) {
+    int l = 0, first = 0;
+    while (j >= a.l[l].end) first = a.l[l++].end;
+    const PrepLayer& p = a.l[l];
+    const int e = (int)j - first;
+    const int ci = e % p.cip, t = (e / p.cip) % 9, co = e / (9 * p.cip);
+    const bool in = co < p.co && ci < p.ci;
+    const uint16_t h = f2bf(in ? p.w[((long)co * p.ci + ci) * 9 + t] : 0.f);
+    p.wf[e] = h;
+    p.wt[((long)ci * 9 + (8 - t)) * p.cop + co] = h;
+    if (ci == 0 && t == 0) p.bp[co] = co < p.co ? p.b[co] : 0.f;
+    return;
+  }
+  for (long i = j - a.nw; i < 2 * a.npix; i += (long)gridDim.x * 256 - a.nw) {
+    const int c0 = (int)(i & 1) * 8;
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = c0 + k < a.C ? a.x[(i >> 1) * a.C + c0 + k] : 0.f;
+    *reinterpret_cast<uint4*>(&a.xb[i * 8]) = pack8(v);
+  }
+}
+
+// The output gradient [npix][C] as bf16 [npix][16], and per block the sums of
+// its channels (the last layer's bias gradient) in double
+__global__ void __launch_bounds__(256) net_gpack_kernel(const float* __restrict__ g, long npix, int C,
+                                                        uint16_t* __restrict__ gb, double* __restrict__ bpart) {
+  __shared__ double sh[4][16];
+  const int tid = threadIdx.x, c0 = (tid & 1) * 8;
+  double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  for (long i = (long)blockIdx.x * 256 + tid; i < 2 * npix; i += (long)gridDim.x * 256) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      v[k] = c0 + k < C ? g[(i >> 1) * C + c0 + k] : 0.f;
+      s[k] += (double)v[k];
+    }
+    *reinterpret_cast<uint4*>(&gb[i * 8]) = pack8(v);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+#pragma unroll
+    for (int d = 2; d < 64; d *= 2) s[k] += __shfl_xor(s[k], d);
+    if ((tid & 63) < 2) sh[tid >> 6][c0 + k] = s[k];
+  }
+  __syncthreads();
+  if (tid < 16) bpart[(long)blockIdx.x * 16 + tid] = ((sh[0][tid] + sh[1][tid]) + sh[2][tid]) + sh[3][tid];
+}
+
+struct SumLayer {
+  const float* part;    // [nch][cop][9][cip]
+  const double* bpart;  // [nb][cop]
+  float* dw;            // (co, ci, ky, kx)
+  float* db;
+  int nch, nb, co, ci, cop, cip;
+  int end;              // blocks of the layers up to this one; the last of a layer sums its biases
+};
+
+struct SumArgs {
+  SumLayer l[TRAIN_L];
+};
+
+// Partial weight and bias gradients of several layers, added in
+// sum_chunks_kernel's order; only the layer's own channels are read, and the
+// weights are written in (co, ci, ky, kx) order
+__global__ void __launch_bounds__(64 * SUM_GROUPS) net_sum_kernel(SumArgs a) {
+  __shared__ double sh[SUM_GROUPS][64];
+  const int e = threadIdx.x & 63, q = threadIdx.x >> 6;
+  int l = 0, first = 0;
+  while ((int)blockIdx.x >= a.l[l].end) first = a.l[l++].end;
+  const SumLayer& p = a.l[l];
+  const bool bias = (int)blockIdx.x == p.end - 1;
+  const int n = bias ? p.co : 9 * p.ci * p.co;
+  const int i = ((int)blockIdx.x - first) * 64 + e, j = bias ? e : i;
+  const int jc = j < n ? j : n - 1;    // in-range address for the spare lanes
+  const int ci = jc % p.ci, t = (jc / p.ci) % 9, co = jc / (9 * p.ci);
+  sh[q][e] = bias ? chunk_sum(p.bpart + jc, p.cop, p.nb, q)
+                  : chunk_sum(p.part + ((long)co * 9 + t) * p.cip + ci, 9L * p.cop * p.cip, p.nch, q);
+  __syncthreads();
+  if (q == 0 && j < n) {
+    double s = sh[0][e];
+#pragma unroll
+    for (int g = 1; g < SUM_GROUPS; ++g) s += sh[g][e];
+    if (bias) p.db[j] = (float)s;
+    else p.dw[((long)co * p.ci + ci) * 9 + t] = (float)s;
+  }
+}
+
+// What a forward pass leaves for the backward pass, in one buffer: the packed
+// input and the activations (bf16), the pre-activations (fp32), the transposed
+// weights, and behind them the forward weights and biases
+struct NetSaved {
+  long npix;
+  int nl;
+  const int* ch;
+  static long up(long b) { return (b + 255) / 256 * 256; }
+  long wbytes(int l) const { return up(2L * 9 * pad16(ch[l]) * pad16(ch[l + 1])); }
+  long act(int l) const {
+    long o = 0;
+    for (int k = 0; k < l; ++k) o += up(2 * npix * pad16(ch[k]));
+    return o;
+  }
+  long z(int l) const {
+    long o = act(nl);
+    for (int k = 0; k < l; ++k) o += up(4 * npix * pad16(ch[k + 1]));
+    return o;
+  }
+  long wt(int l) const {
+    long o = z(nl - 1);
+    for (int k = 0; k < l; ++k) o += wbytes(k);
+    return o;
+  }
+  long wf(int l) const { return wt(nl) + wt(l) - wt(0); }
+  long bp(int l) const {
+    long o = wf(nl);
+    for (int k = 0; k < l; ++k) o += up(4L * pad16(ch[k + 1]));
+    return o;
+  }
+  long bytes() const { return bp(nl); }
+};
+
+constexpr int WGRAD_CHUNKS = 512;         // as many partial weight gradients
+constexpr long PART_BYTES = 128L << 20;   // partials of several layers up to this wait for one summing launch
+constexpr int GPACK_BLOCKS = 512;
+
+// Backward scratch: two bf16 gradients, an fp32 one where a layer's shape
+// needs the separate column sums, partial bias and weight gradients
+struct NetScratch {
+  long npix;
+  int B, H, W, nl;
+  const int* ch;
+  static long up(long b) { return NetSaved::up(b); }
+  int cmax() const {
+    int c = 0;
+    for (int l = 1; l <= nl; ++l) c = pad16(ch[l]) > c ? pad16(ch[l]) : c;
+    return c;
+  }
+  // tile width of the convolution that gives the gradient at layer l's output
+  int dgrad_tc(int l) const { return tile_cols(H, W, pad16(ch[l + 2]), pad16(ch[l + 1])); }
+  long dz(int k) const { return k * up(2 * npix * cmax()); }
+  long dzf() const { return dz(2); }
+  long bpart(int k) const {
+    long c = 0;
+    for (int l = 0; l < nl - 1; ++l) {
+      if (!dgrad_tc(l) && pad16(ch[l + 1]) > c) c = pad16(ch[l + 1]);
+    }
+    return dzf() + up(4 * npix * c) + k * (1024L * 8 * 64);
+  }
+  long part() const { return bpart(TRAIN_L); }
+  int nchunk() const {
+    const long n = npix / 256;
+    return (int)(n < 1 ? 1 : n < WGRAD_CHUNKS ? n : WGRAD_CHUNKS);
+  }
+  long pbytes(int l) const { return up(4L * nchunk() * 9 * pad16(ch[l]) * pad16(ch[l + 1])); }
+  long part_bytes() const {
+    long sum = 0, one = 0;
+    for (int l = 0; l < nl; ++l) {
+      sum += pbytes(l);
+      one = pbytes(l) > one ? pbytes(l) : one;
+    }
+    return sum < PART_BYTES ? sum : one > PART_BYTES ? one : PART_BYTES;
+  }
+  long bytes() const { return part() + part_bytes(); }
+};
+
+int check_net(int B, int H, int W, int nl, const int* ch) {
+  if (!ch || nl < 1) return ddx::set_error(DDX_ERR_ARG, "bad network");
+  for (int l = 0; l <= nl; ++l)
+    if (ch[l] < 1) return ddx::set_error(DDX_ERR_ARG, "bad network channels");
+  if (ch[0] > DDX_CONV_MAXCH) return ddx::set_error(DDX_ERR_ARG, "at most 16 input channels");
+  for (int l = 0; l < nl; ++l) {
+    const int rc = check_conv(B, H, W, pad16(ch[l]), pad16(ch[l + 1]));
+    if (rc) return rc;
+  }
+  return 0;
+}
+
 // ---------------------------------------------------------------------------
 // The whole network in one launch (inference)
 // ---------------------------------------------------------------------------
@@ -942,12 +1331,6 @@ __device__ inline int wrapm(int i, int n) {
 // global memory once per tile, not once per wavefront.  load() runs a layer
 // ahead, under the previous layer's arithmetic; the bias stays in registers
 // (a lane's four output channels of each 16).
-__device__ inline bf16x8 lds16(const uint16_t* p) {
-  const uint4 v = *reinterpret_cast<const uint4*>(p);
-  const u32x4 u = {v.x, v.y, v.z, v.w};
-  return __builtin_bit_cast(bf16x8, u);
-}
-
 template <int CI, int CO, int NT>
 struct NetStage {
   static constexpr int NCO = CO / 16, KQ = CI == 32 ? 8 : 4;
@@ -1551,48 +1934,7 @@ extern "C" {
 
 int ddx_conv3x3(void* stream, int B, int H, int W, int Ci, int Co, const void* x, const void* w,
                 const float* bias, const float* aux, int mode, float* out_f32, void* out_bf16) {
-  int rc = check_conv(B, H, W, Ci, Co);
-  if (rc) return rc;
-  if (!x || !w || (!out_f32 && !out_bf16)) return ddx::set_error(DDX_ERR_ARG, "null argument");
-  if (mode != DDX_CONV_LINEAR && mode != DDX_CONV_GELU && mode != DDX_CONV_GELU_GRAD)
-    return ddx::set_error(DDX_ERR_ARG, "unknown convolution mode");
-  if (mode == DDX_CONV_GELU_GRAD && !aux)
-    return ddx::set_error(DDX_ERR_ARG, "DDX_CONV_GELU_GRAD needs the pre-activation");
-  ConvArgs a{(const uint16_t*)x, (const uint16_t*)w, bias, aux, out_f32, (uint16_t*)out_bf16,
-             B, H, W, Ci, Co, mode};
-  hipStream_t s = (hipStream_t)stream;
-  auto al = [](const void* q, uintptr_t n) { return ((uintptr_t)q % n) == 0; };
-  const bool aligned = al(x, 16) && al(w, 16) && al(out_f32, 16) && al(aux, 16) && al(out_bf16, 8);
-  if (aligned && W % 64 == 0 && H % 4 == 0 && (Ci == 16 || Ci == 32) && (Co == 16 || Co == 32)) {
-    // blocks loop over tiles; about four resident blocks per CU cover the chip
-    const long ntiles = (long)B * (H / 4) * (W / 64);
-    const dim3 tgrid((unsigned)(ntiles < 1024 ? ntiles : 1024));
-    const int key = Ci * 100 + Co;
-    // bf16-only output without the GELU gradient stages bf16 (BF)
-    if (!out_f32 && mode != DDX_CONV_GELU_GRAD) {
-      if (key == 1616) hipLaunchKernelGGL((conv3x3_tile_kernel<16, 16, true>), tgrid, dim3(256), 0, s, a, ntiles);
-      else if (key == 1632) hipLaunchKernelGGL((conv3x3_tile_kernel<16, 32, true>), tgrid, dim3(256), 0, s, a, ntiles);
-      else if (key == 3216) hipLaunchKernelGGL((conv3x3_tile_kernel<32, 16, true>), tgrid, dim3(256), 0, s, a, ntiles);
-      else hipLaunchKernelGGL((conv3x3_tile_kernel<32, 32, true>), tgrid, dim3(256), 0, s, a, ntiles);
-    } else {
-      if (key == 1616) hipLaunchKernelGGL((conv3x3_tile_kernel<16, 16, false>), tgrid, dim3(256), 0, s, a, ntiles);
-      else if (key == 1632) hipLaunchKernelGGL((conv3x3_tile_kernel<16, 32, false>), tgrid, dim3(256), 0, s, a, ntiles);
-      else if (key == 3216) hipLaunchKernelGGL((conv3x3_tile_kernel<32, 16, false>), tgrid, dim3(256), 0, s, a, ntiles);
-      else hipLaunchKernelGGL((conv3x3_tile_kernel<32, 32, false>), tgrid, dim3(256), 0, s, a, ntiles);
-    }
-    CL_LAUNCHCHK("conv3x3 tile");
-    return 0;
-  }
-  const long tiles = (long)B * H * W / 16;
-  const dim3 grid(nblk(tiles, 4));
-  switch (Co / 16) {
-    case 1: hipLaunchKernelGGL(conv3x3_kernel<1>, grid, dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL(conv3x3_kernel<2>, grid, dim3(256), 0, s, a); break;
-    case 3: hipLaunchKernelGGL(conv3x3_kernel<3>, grid, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL(conv3x3_kernel<4>, grid, dim3(256), 0, s, a); break;
-  }
-  CL_LAUNCHCHK("conv3x3");
-  return 0;
+  return conv_run((hipStream_t)stream, B, H, W, Ci, Co, x, w, bias, aux, mode, out_f32, out_bf16, Co);
 }
 
 int ddx_conv3x3_wgrad(void* stream, int B, int H, int W, int Ci, int Co, const void* x,
@@ -1602,24 +1944,11 @@ int ddx_conv3x3_wgrad(void* stream, int B, int H, int W, int Ci, int Co, const v
   if (!x || !dz || !partial || !dw || nchunk < 1) return ddx::set_error(DDX_ERR_ARG, "null argument");
   const long npix = (long)B * H * W;
   hipStream_t s = (hipStream_t)stream;
-  if (W % 64 == 0 && H % 4 == 0 && (Ci == 16 || Ci == 32) && (Co == 16 || Co == 32)) {
-    const long ntiles = (long)B * (H / 4) * (W / 64);
-    const int nch = (int)(ntiles < nchunk ? ntiles : nchunk);
-    const int key = Ci * 100 + Co;
-    if (key == 1616)
-      hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<16, 16>), dim3(nch), dim3(256), 0, s,
-                         (const uint16_t*)x, (const uint16_t*)dz, partial, B, H, W);
-    else if (key == 1632)
-      hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<16, 32>), dim3(nch), dim3(256), 0, s,
-                         (const uint16_t*)x, (const uint16_t*)dz, partial, B, H, W);
-    else if (key == 3216)
-      hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<32, 16>), dim3(nch), dim3(256), 0, s,
-                         (const uint16_t*)x, (const uint16_t*)dz, partial, B, H, W);
-    else
-      hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<32, 32>), dim3(nch), dim3(256), 0, s,
-                         (const uint16_t*)x, (const uint16_t*)dz, partial, B, H, W);
+  const long n = (long)Co * 9 * Ci;
+  const int tc = tile_cols(H, W, Ci, Co);
+  if (tc) {
+    const int nch = wgrad_tiles(s, B, H, W, Ci, Co, tc, x, dz, nullptr, partial, nullptr, nchunk);
     CL_LAUNCHCHK("conv3x3_wgrad tile");
-    const long n = (long)Co * 9 * Ci;
     hipLaunchKernelGGL(sum_chunks_kernel, dim3(nblk(n, 64)), dim3(64 * SUM_GROUPS), 0, s, partial, dw, nch, n);
     CL_LAUNCHCHK("conv3x3_wgrad sum");
     return 0;
@@ -1630,7 +1959,6 @@ int ddx_conv3x3_wgrad(void* stream, int B, int H, int W, int Ci, int Co, const v
   hipLaunchKernelGGL(conv3x3_wgrad_kernel, dim3(nch, (Co / 16) * (Ci / 16)), dim3(64), 0, s,
                      (const uint16_t*)x, (const uint16_t*)dz, partial, B, H, W, Ci, Co, (int)pch);
   CL_LAUNCHCHK("conv3x3_wgrad");
-  const long n = (long)Co * 9 * Ci;
   hipLaunchKernelGGL(sum_chunks_kernel, dim3(nblk(n, 64)), dim3(64 * SUM_GROUPS), 0, s, partial, dw, nch, n);
   CL_LAUNCHCHK("conv3x3_wgrad sum");
   return 0;
@@ -1647,23 +1975,7 @@ int ddx_conv3x3_grads(void* stream, int B, int H, int W, int Ci, int Co, const v
     return ddx::set_error(DDX_ERR_UNSUPPORTED,
                           "fused gradients need W % 64 == 0, H % 4 == 0 and 16 or 32 channels");
   hipStream_t s = (hipStream_t)stream;
-  const long ntiles = (long)B * (H / 4) * (W / 64);
-  const int nch = (int)(ntiles < nchunk ? ntiles : nchunk);
-  const int key = Ci * 100 + Co;
-  const uint16_t* xx = (const uint16_t*)x;
-  const uint16_t* dd = (const uint16_t*)dz;
-  if (key == 1616)
-    hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<16, 16>), dim3(nch), dim3(256), 0, s, xx, dd, partial,
-                       B, H, W, dzf, bpartial);
-  else if (key == 1632)
-    hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<16, 32>), dim3(nch), dim3(256), 0, s, xx, dd, partial,
-                       B, H, W, dzf, bpartial);
-  else if (key == 3216)
-    hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<32, 16>), dim3(nch), dim3(256), 0, s, xx, dd, partial,
-                       B, H, W, dzf, bpartial);
-  else
-    hipLaunchKernelGGL((conv3x3_wgrad_tile_kernel<32, 32>), dim3(nch), dim3(256), 0, s, xx, dd, partial,
-                       B, H, W, dzf, bpartial);
+  const int nch = wgrad_tiles(s, B, H, W, Ci, Co, 64, x, dz, dzf, partial, bpartial, nchunk);
   CL_LAUNCHCHK("conv3x3 grads");
   const long n = (long)Co * 9 * Ci;
   hipLaunchKernelGGL(sum_chunks_kernel, dim3(nblk(n, 64)), dim3(64 * SUM_GROUPS), 0, s, partial, dw, nch, n);
@@ -1861,6 +2173,139 @@ int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
   return ddx::set_error(DDX_ERR_UNSUPPORTED,
                         "fused network: depth 5 width 32 on images of multiples of 8 x 8 "
                         "pixels, or depth 3 width 16 on multiples of 8 x 16");
+}
+
+int ddx_net_bytes(int B, int H, int W, int nl, const int* chans, int64_t* saved, int64_t* scratch) {
+  int rc = check_net(B, H, W, nl, chans);
+  if (rc) return rc;
+  if (!saved || !scratch) return ddx::set_error(DDX_ERR_ARG, "null argument");
+  const long npix = (long)B * H * W;
+  *saved = NetSaved{npix, nl, chans}.bytes();
+  *scratch = NetScratch{npix, B, H, W, nl, chans}.bytes();
+  return 0;
+}
+
+int ddx_net_forward(void* stream, int B, int H, int W, int nl, const int* chans, const float* x,
+                    const float* const* w, const float* const* bias, void* saved, float* out) {
+  int rc = check_net(B, H, W, nl, chans);
+  if (rc) return rc;
+  if (!x || !w || !bias || !saved || !out) return ddx::set_error(DDX_ERR_ARG, "null argument");
+  if ((uintptr_t)saved % 16) return ddx::set_error(DDX_ERR_ARG, "the saved buffer must be 16-byte aligned");
+  for (int l = 0; l < nl; ++l)
+    if (!w[l] || !bias[l]) return ddx::set_error(DDX_ERR_ARG, "null argument");
+  hipStream_t s = (hipStream_t)stream;
+  const long npix = (long)B * H * W;
+  const NetSaved m{npix, nl, chans};
+  char* base = (char*)saved;
+  auto act = [&](int l) { return (uint16_t*)(base + m.act(l)); };
+  for (int l0 = 0; l0 < nl; l0 += TRAIN_L) {
+    PrepArgs a{};
+    a.nl = nl - l0 < TRAIN_L ? nl - l0 : TRAIN_L;
+    for (int k = 0; k < a.nl; ++k) {
+      const int l = l0 + k, co = chans[l + 1], ci = chans[l];
+      a.nw += 9 * pad16(ci) * pad16(co);
+      a.l[k] = PrepLayer{w[l], bias[l], (uint16_t*)(base + m.wf(l)), (uint16_t*)(base + m.wt(l)),
+                         (float*)(base + m.bp(l)), co, ci, pad16(co), pad16(ci), a.nw};
+    }
+    if (l0 == 0) {
+      a.x = x;
+      a.xb = act(0);
+      a.npix = npix;
+      a.C = chans[0];
+    }
+    const long items = 2 * a.npix < (1L << 28) ? 2 * a.npix : 1L << 28;   // a loop covers more
+    hipLaunchKernelGGL(net_prep_kernel, dim3(nblk(a.nw + items, 256)), dim3(256), 0, s, a);
+    CL_LAUNCHCHK("net_forward: prepare");
+  }
+  for (int l = 0; l < nl; ++l) {
+    const bool last = l == nl - 1;
+    rc = conv_run(s, B, H, W, pad16(chans[l]), pad16(chans[l + 1]), act(l), base + m.wf(l),
+                  (const float*)(base + m.bp(l)), nullptr, last ? DDX_CONV_LINEAR : DDX_CONV_GELU,
+                  last ? out : (float*)(base + m.z(l)), last ? nullptr : act(l + 1),
+                  last ? chans[nl] : pad16(chans[l + 1]));
+    if (rc) return rc;
+  }
+  return 0;
+}
+
+int ddx_net_backward(void* stream, int B, int H, int W, int nl, const int* chans, const float* g,
+                     const void* saved, void* scratch, float* const* dw, float* const* db) {
+  int rc = check_net(B, H, W, nl, chans);
+  if (rc) return rc;
+  if (!g || !saved || !scratch || !dw || !db) return ddx::set_error(DDX_ERR_ARG, "null argument");
+  if (chans[nl] > DDX_CONV_MAXCH) return ddx::set_error(DDX_ERR_ARG, "at most 16 output channels");
+  if ((uintptr_t)saved % 16 || (uintptr_t)scratch % 16)
+    return ddx::set_error(DDX_ERR_ARG, "the saved and scratch buffers must be 16-byte aligned");
+  for (int l = 0; l < nl; ++l)
+    if (!dw[l] || !db[l]) return ddx::set_error(DDX_ERR_ARG, "null argument");
+  hipStream_t s = (hipStream_t)stream;
+  const long npix = (long)B * H * W;
+  const NetSaved m{npix, nl, chans};
+  const NetScratch t{npix, B, H, W, nl, chans};
+  const char* base = (const char*)saved;
+  char* sc = (char*)scratch;
+  SumArgs sums{};
+  int ns = 0;
+  long used = 0;
+  uint16_t* dz = (uint16_t*)(sc + t.dz(0));
+  // nb partial column sums of layer l's output gradient, in bpart slot ns
+  const long gb = (2 * npix + 255) / 256;
+  int nb = (int)(gb < GPACK_BLOCKS ? gb : GPACK_BLOCKS);
+  hipLaunchKernelGGL(net_gpack_kernel, dim3(nb), dim3(256), 0, s, g, npix, chans[nl], dz, (double*)(sc + t.bpart(0)));
+  CL_LAUNCHCHK("net_backward: pack");
+  for (int l = nl - 1; l >= 0; --l) {
+    const int cip = pad16(chans[l]), cop = pad16(chans[l + 1]);
+    const uint16_t* x = (const uint16_t*)(base + m.act(l));
+    float* part = (float*)(sc + t.part() + used);
+    int nch = t.nchunk();
+    const int tc = tile_cols(H, W, cip, cop);
+    if (tc) {
+      nch = wgrad_tiles(s, B, H, W, cip, cop, tc, x, dz, nullptr, part, nullptr, nch);
+    } else {
+      long pch = (npix + nch - 1) / nch;
+      pch = (pch + 15) / 16 * 16;
+      nch = (int)((npix + pch - 1) / pch);
+      hipLaunchKernelGGL(conv3x3_wgrad_kernel, dim3(nch, (cop / 16) * (cip / 16)), dim3(64), 0, s, x, dz, part, B, H, W,
+                         cip, cop, (int)pch);
+    }
+    CL_LAUNCHCHK("net_backward: weight gradient");
+    const int blocks = (int)nblk(9L * chans[l] * chans[l + 1], 64) + 1;
+    sums.l[ns] = SumLayer{part, (const double*)(sc + t.bpart(ns)), dw[l], db[l], nch, nb, chans[l + 1], chans[l],
+                          cop, cip, (ns ? sums.l[ns - 1].end : 0) + blocks};
+    ++ns;
+    used += t.pbytes(l);
+    if (l == 0 || ns == TRAIN_L || used + t.pbytes(l - 1) > t.part_bytes()) {
+      hipLaunchKernelGGL(net_sum_kernel, dim3(sums.l[ns - 1].end), dim3(64 * SUM_GROUPS), 0, s, sums);
+      CL_LAUNCHCHK("net_backward: sums");
+      ns = 0;
+      used = 0;
+    }
+    if (l == 0) break;
+    // the gradient at layer l - 1's output
+    uint16_t* dn = (uint16_t*)(sc + t.dz((nl - l) & 1));
+    const float* z = (const float*)(base + m.z(l - 1));
+    const int dtc = t.dgrad_tc(l - 1);
+    if (dtc) {
+      const ConvArgs a{dz, (const uint16_t*)(base + m.wt(l)), nullptr, z, nullptr, dn, B, H, W, cop, cip,
+                       DDX_CONV_GELU_GRAD, cip, (double*)(sc + t.bpart(ns))};
+      conv_tile<false>(s, a, dtc);
+      CL_LAUNCHCHK("net_backward: input gradient");
+      nb = (int)conv_blocks(npix / 256);
+    } else {
+      float* dzf = (float*)(sc + t.dzf());
+      double* bp = (double*)(sc + t.bpart(ns));
+      rc = conv_run(s, B, H, W, cop, cip, dz, base + m.wt(l), nullptr, z, DDX_CONV_GELU_GRAD, dzf, dn, cip);
+      if (rc) return rc;
+      const long nc = npix / 1024 < 1 ? 1 : npix / 1024 < 1024 ? npix / 1024 : 1024;
+      const long chunk = (npix + nc - 1) / nc;
+      const int nblocks = (int)((npix + chunk - 1) / chunk);
+      hipLaunchKernelGGL(colsum_partial_kernel, dim3(nblocks), dim3(256), 0, s, dzf, bp, npix, cip, chunk);
+      CL_LAUNCHCHK("net_backward: column sums");
+      nb = nblocks;
+    }
+    dz = dn;
+  }
+  return 0;
 }
 
 int ddx_mfma_probe(void* stream, int k, const void* A, const void* Bm, float* D) {

@@ -5,14 +5,13 @@ multiple of 16; the network's own input and output are [B, H, W, C] float32
 tensors on the GPU.  Every layer is a 3x3 periodic convolution; hidden
 layers apply GELU (tanh form, z sigma(2 sqrt(2/pi) (z + 0.044715 z^3))).  Weights and biases are float32
 torch Parameters in torch's (co, ci, ky, kx) layout; each forward pass
-rounds them to bf16 once (``ddx_conv_wprep``) and every product
-accumulates in float32.
+rounds them to bf16 once and every product accumulates in float32.
 
 Forward of layer l:   z_l = conv(a_{l-1}, w_l) + b_l,  a_l = bf16(GELU(z_l))
-Backward of layer l:  dW_l = sum_p bf16(dz_l) x shift(a_{l-1})   (ddx_conv3x3_wgrad)
-                      db_l = sum_p dz_l                          (ddx_conv_colsum)
+Backward of layer l:  dW_l = sum_p bf16(dz_l) x shift(a_{l-1})
+                      db_l = sum_p dz_l
                       dz_{l-1} = conv(bf16(dz_l), w_l^T) * GELU'(z_{l-1})
-                                                    (one ddx_conv3x3 call, fused)
+all layers in one native call each way (ddx_net_forward, ddx_net_backward).
 """
 
 import ctypes
@@ -193,66 +192,73 @@ def unpack(src, C, dsts, f64, pstride=1, scale=None, add=None):
                                1 if f64 else 0, sc, ad))
 
 
+def _param(p, shape, dev):
+    """A parameter as the contiguous float32 tensor of this shape that the
+    kernels read: a smaller weight is padded with zeros, a bias broadcast."""
+    if p.shape == shape and p.dtype == torch.float32 and p.device == dev and p.is_contiguous():
+        return p
+    p = p.detach().to(device=dev, dtype=torch.float32)
+    if p.shape != shape:
+        if len(shape) == 1:
+            p = p.expand(shape)
+        elif p.dim() != 4 or p.shape[2:] != (3, 3) or p.shape[0] > shape[0] or p.shape[1] > shape[1]:
+            raise ValueError("closure weights of shape %s do not fit a layer of %s" % (tuple(p.shape), shape))
+        else:
+            p = torch.nn.functional.pad(p, (0, 0, 0, 0, 0, shape[1] - p.shape[1], 0, shape[0] - p.shape[0]))
+    return p.contiguous()
+
+
+def _chans(chans):
+    return (ctypes.c_int * len(chans))(*chans)
+
+
 class _NetFn(torch.autograd.Function):
-    """The whole network as one autograd node, so the GELU derivative of each
+    """The whole network as one autograd node and one native call each way
+    (``ddx_net_forward``, ``ddx_net_backward``): the GELU derivative of each
     layer fuses into the next input-gradient convolution."""
 
     @staticmethod
     def forward(ctx, x, chans, *params):
         nl = len(chans) - 1
-        ws, bs = params[:nl], params[nl:]
         B, H, W, cin = x.shape
-        npix = B * H * W
-        assert cin == chans[0] and npix % 16 == 0
+        assert cin == chans[0] and B * H * W % 16 == 0
+        lib = _lib()
+        dev = x.device
+        ch = _chans(chans)
+        nsaved, nscratch = ctypes.c_int64(), ctypes.c_int64()
+        _check(lib.ddx_net_bytes(B, H, W, nl, ch, nsaved, nscratch))
         xc = x.detach().contiguous()
-        a, _ = pack([(xc.data_ptr() + 4 * c, False) for c in range(cin)], npix, pad16(cin),
-                    pstride=cin)
-        acts, zs, wts = [a], [], []
-        out = None
-        for l in range(nl):
-            ci, co = chans[l], chans[l + 1]
-            cip, cop = pad16(ci), pad16(co)
-            wf, wt = wprep(ws[l], cop, cip)
-            bp = torch.zeros(cop, dtype=torch.float32, device=x.device)
-            bp[:co] = bs[l].detach()
-            wts.append(wt)
-            if l < nl - 1:
-                z, a = conv3x3(acts[-1], wf, B, H, W, bias=bp, mode=_hip.CONV_GELU,
-                               out_f32=True, out_bf16=True)
-                zs.append(z)
-                acts.append(a)
-            else:
-                out, _ = conv3x3(acts[-1], wf, B, H, W, bias=bp, mode=_hip.CONV_LINEAR)
+        ws = [_param(params[l], (chans[l + 1], chans[l], 3, 3), dev) for l in range(nl)]
+        bs = [_param(params[nl + l], (chans[l + 1],), dev) for l in range(nl)]
+        saved = torch.empty(nsaved.value, dtype=torch.uint8, device=dev)
+        out = torch.empty((B, H, W, chans[-1]), dtype=torch.float32, device=dev)
+        _check(lib.ddx_net_forward(_stream(), B, H, W, nl, ch, _ptr(xc),
+                                   _hip.ptr_array([p.data_ptr() for p in ws]),
+                                   _hip.ptr_array([p.data_ptr() for p in bs]),
+                                   _ptr(saved), _ptr(out)))
         ctx.chans = chans
         ctx.shape = (B, H, W)
-        ctx.save_for_backward(*acts, *zs, *wts)
-        return out[:, :chans[-1]].reshape(B, H, W, chans[-1])
+        ctx.nscratch = nscratch.value
+        ctx.save_for_backward(saved)
+        return out
 
     @staticmethod
     def backward(ctx, g):
         chans = ctx.chans
         nl = len(chans) - 1
         B, H, W = ctx.shape
-        npix = B * H * W
-        saved = ctx.saved_tensors
-        acts, zs, wts = saved[:nl], saved[nl:2 * nl - 1], saved[2 * nl - 1:]
+        saved, = ctx.saved_tensors
+        if not saved.is_contiguous() or saved.data_ptr() % 16:
+            saved = saved.clone(memory_format=torch.contiguous_format)
         gc = g.detach().contiguous()
-        cout = chans[-1]
-        dzb, dzf = pack([(gc.data_ptr() + 4 * c, False) for c in range(cout)], npix,
-                        pad16(cout), pstride=cout, bf16=True, f32=True)
-        gws, gbs = [None] * nl, [None] * nl
-        for l in range(nl - 1, -1, -1):
-            ci, co = chans[l], chans[l + 1]
-            g2 = grads(acts[l], dzb, dzf, B, H, W)
-            if g2 is None:
-                gws[l] = wunpack(wgrad(acts[l], dzb, B, H, W), co, ci)
-                gbs[l] = colsum(dzf)[:co].contiguous()
-            else:
-                gws[l] = wunpack(g2[0], co, ci)
-                gbs[l] = g2[1][:co].contiguous()
-            if l > 0:
-                dzf, dzb = conv3x3(dzb, wts[l], B, H, W, aux=zs[l - 1],
-                                   mode=_hip.CONV_GELU_GRAD, out_f32=True, out_bf16=True)
+        dev = gc.device
+        scratch = torch.empty(ctx.nscratch, dtype=torch.uint8, device=dev)
+        gws = [torch.empty((chans[l + 1], chans[l], 3, 3), dtype=torch.float32, device=dev)
+               for l in range(nl)]
+        gbs = [torch.empty(chans[l + 1], dtype=torch.float32, device=dev) for l in range(nl)]
+        _check(_lib().ddx_net_backward(_stream(), B, H, W, nl, _chans(chans), _ptr(gc), _ptr(saved),
+                                       _ptr(scratch), _hip.ptr_array([t.data_ptr() for t in gws]),
+                                       _hip.ptr_array([t.data_ptr() for t in gbs])))
         return (None, None, *gws, *gbs)
 
 
@@ -280,7 +286,9 @@ class ClosureNet(torch.nn.Module):
             raise _hip.DDXError(-5, "ClosureNet runs on the HIP kernels only (input is on the CPU)")
         if x.dtype != torch.float32 or x.dim() != 4 or x.shape[-1] != self.chans[0]:
             raise ValueError("ClosureNet input must be float32 [B, H, W, %d]" % self.chans[0])
-        return _NetFn.apply(x, self.chans, *self.weights, *self.biases)
+        keys = [str(l) for l in range(len(self.chans) - 1)]   # ParameterList's own names
+        return _NetFn.apply(x, self.chans, *[getattr(self.weights, k) for k in keys],
+                            *[getattr(self.biases, k) for k in keys])
 
     def flops_per_pixel(self):
         """Multiply-adds x 2 per pixel of one forward pass, padded channels."""

@@ -45,9 +45,9 @@ enum { DDX_CONV_MAXCH = 16 }; /* channels per pack / unpack call */
  * aux [npix][Co] fp32 (GELU_GRAD only).  Writes out_f32 [npix][Co] and/or
  * out_bf16 [npix][Co] (either may be NULL, not both).  With the transposed
  * weights of ddx_conv_wprep, the same call gives the input gradient.
- * Widths W % 64 == 0, heights H % 4 == 0 and 16 or 32 channels with 16-byte
- * aligned x, w, out_f32, aux (8-byte aligned out_bf16) take the LDS-tiled
- * kernel; other shapes a per-fragment kernel with the same results. */
+ * Widths W % 64 == 0 with heights H % 4 == 0, or W % 32 == 0 with H % 8 == 0,
+ * and 16 or 32 channels with 16-byte aligned x, w, out_f32, aux (8-byte
+ * aligned out_bf16) take the LDS-tiled kernel; other shapes a per-fragment kernel with the same results. */
 int ddx_conv3x3(void* stream, int B, int H, int W, int Ci, int Co, const void* x, const void* w,
                 const float* bias, const float* aux, int mode, float* out_f32, void* out_bf16);
 
@@ -127,6 +127,23 @@ int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
                  const void* const* w, const float* const* bias, const void* x, float* out,
                  const void* const* src, const float* in_scale, void* const* dst,
                  const void* const* add, const float* out_scale);
+
+/* Training.  The network of ddx_conv_net's description with any depth and
+ * widths ddx_conv3x3 takes (inputs of at most 16 channels): ddx_net_forward
+ * gives out [npix][chans[nl]] fp32 from x [npix][chans[0]] fp32 and the fp32
+ * parameters w[l] (co, ci, ky, kx) and bias[l] (co), and leaves in saved what
+ * the backward pass needs: bf16 activations, fp32 pre-activations and the
+ * transposed weights, so the parameters may change in between.
+ * ddx_net_backward turns g = dL/dout [npix][chans[nl]] (at most 16 channels)
+ * into dw[l], db[l] in the parameters' layouts, with the arithmetic of
+ * ddx_conv3x3_wgrad, ddx_conv_colsum and ddx_conv3x3 (GELU_GRAD).
+ * ddx_net_bytes gives the sizes of the saved and the scratch buffer, both
+ * 16-byte aligned. */
+int ddx_net_bytes(int B, int H, int W, int nl, const int* chans, int64_t* saved, int64_t* scratch);
+int ddx_net_forward(void* stream, int B, int H, int W, int nl, const int* chans, const float* x,
+                    const float* const* w, const float* const* bias, void* saved, float* out);
+int ddx_net_backward(void* stream, int B, int H, int W, int nl, const int* chans, const float* g,
+                     const void* saved, void* scratch, float* const* dw, float* const* db);
 
 /* Layout check: D = A B for one 16 x 16 x k bf16 tile (k = 16 or 32) on one
  * wavefront, with the lane placement the convolution kernels use (A 16 x k,

@@ -22,11 +22,14 @@ bool mix_col_launch(hipStream_t s, ColArgs<T>& a, const MixPlan& mp0, int nslabs
   // 32-bit byte offsets from the start of a slab, where they reach
   const size_t lim = ((size_t)1 << 32) / sizeof(cpx<T>);
   const bool big = (size_t)a.in_rows * a.in_rs + a.ncols >= lim || (size_t)a.out_rows * a.out_rs + a.ncols >= lim;
-  // Tile width: whole 256-byte rows within 48 KB of LDS (three workgroups
-  // per CU), then narrower down to 64 bytes while the launch would leave
-  // CUs without a workgroup.
-  const int wmax = 256 / (int)sizeof(cpx<T>), wmin = 64 / (int)sizeof(cpx<T>);
-  int W = wmax;
+  // Tile width: 16 columns within 48 KB of LDS (three workgroups per CU),
+  // then narrower down to 64 bytes while the launch would leave CUs without a
+  // workgroup.  Eight FP64 columns cost 4 % at 192^3 (60.0 against 57.7 us,
+  // spectral passes); 32 FP32 columns cost 15-30 % (128^3: 20.5 against 15.5
+  // us spectral; 256 members 128^2: 23.6 against 19.9), a third of it lanes
+  // past the last column of 48.
+  const int wmin = 64 / (int)sizeof(cpx<T>);
+  int W = 16;
   while (W > 1 && (size_t)n * W * sizeof(cpx<T>) > 49152) W /= 2;
   while (W > wmin && (long)((a.ncols + W - 1) / W) * nslabs * nfields < 512) W /= 2;
   if ((size_t)n * W * sizeof(cpx<T>) > 65536) return false;

@@ -190,10 +190,12 @@ __device__ inline bf16x8 lds8(const uint16_t* p) {
 // c + gridDim.x, ...): the weights are staged in LDS once per block, and the
 // next tile's input halo is loaded into registers while the current tile
 // computes.  The first halo and, for the GELU gradient, a tile's
-// pre-activations are requested before anything waits: with one tile per
-// block (a training batch of 32 images 64^2) the kernel is a chain of memory
-// latencies.  TC = 32 multiplies 32 channels in two steps of 16, the sums of
-// conv3x3_kernel.  Pixel stride and weight-row stride CI + 4 (bf16) place the
+// pre-activations are requested before anything waits.  A training batch of
+// 32 images 64^2 (one tile per block) takes 12.8 us per 32-channel layer, the
+// larger part of it the 24 MB of fp32 and bf16 stores: stored straight from
+// the accumulators, in 64-byte pieces instead of the staging's whole lines,
+// it took 13.8.  TC = 32 multiplies 32 channels in two steps of 16, the sums
+// of conv3x3_kernel.  Pixel stride and weight-row stride CI + 4 (bf16) place the
 // 16 rows of a fragment read in distinct bank pairs.  CI = 32 uses the
 // gfx950 16x16x32 bf16 MFMA, CI = 16 the 16x16x16 one.
 //
@@ -1735,24 +1737,14 @@ __device__ __forceinline__ void rn_hidden(unsigned char* lds, const int (&out)[2
 
 // An input row y (wrapped), 32 bytes of 16 bf16 channels per pixel: thread
 // tid < 2 W of group 0 brings half tid & 1 of pixel tid >> 1
-template <int W, bool FIELDS>
+template <int W>
 struct RowInput {
   uint4 q;
   __device__ __forceinline__ void load(const NetArgs& a, int b, int y, int tid) {
     if (tid >= 2 * W) return;
     const int p = tid >> 1, h = tid & 1;
     const long gp = ((long)b * a.H + wrapm(y, a.H)) * W + p;
-    if (!FIELDS) {
-      q = *reinterpret_cast<const uint4*>(&a.x[gp * 16 + 8 * h]);
-    } else {
-      float v[8];
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const int ch = 8 * h + c, cc = ch < a.cin ? ch : 0;
-        v[c] = ch < a.cin ? (float)a.src[cc][gp] * a.in_scale[cc] : 0.f;
-      }
-      q = make_uint4(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]), f2bf2(v[4], v[5]), f2bf2(v[6], v[7]));
-    }
+    q = *reinterpret_cast<const uint4*>(&a.x[gp * 16 + 8 * h]);
   }
   __device__ __forceinline__ void store(unsigned char* row, int tid) const {
     if (tid >= 2 * W) return;
@@ -1775,7 +1767,7 @@ __device__ __forceinline__ void rn_interleave() {
   }
 }
 
-template <int W, bool FIELDS>
+template <int W>
 __global__ void __launch_bounds__(RowNet<W>::NT, 4) conv_rows_kernel(NetArgs a, int S, int strips) {
   using P = RowNet<W>;
   constexpr int HROW = P::HROW, IROW = P::IROW;
@@ -1803,7 +1795,7 @@ __global__ void __launch_bounds__(RowNet<W>::NT, 4) conv_rows_kernel(NetArgs a, 
     }
     // group 0 also brings the input: rows y0 - 5 .. y0 - 3 before the first
     // step, then one a step, loaded a step ahead
-    RowInput<W, FIELDS> in;
+    RowInput<W> in;
 #pragma unroll 1
     for (int r = 0; r < 3; ++r) {
       in.load(a, b, y0 - 5 + r, tid);
@@ -1835,18 +1827,7 @@ __global__ void __launch_bounds__(RowNet<W>::NT, 4) conv_rows_kernel(NetArgs a, 
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = oc[i] + b4[i];
-        if (!FIELDS) {
-          *reinterpret_cast<float4*>(&a.out[gp * 16 + 4 * kq]) = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int co = 4 * kq + i;
-            if (co < a.cout) {
-              const float x = v[i] * a.out_scale[co];
-              a.dst[co][gp] = (double)x + (a.add[0] ? a.add[co][gp] : 0.0);
-            }
-          }
-        }
+        *reinterpret_cast<float4*>(&a.out[gp * 16 + 4 * kq]) = make_float4(v[0], v[1], v[2], v[3]);
       }
       __builtin_amdgcn_sched_barrier(0);
       rn_conv<16, 32, IROW, PH>(rnlds, off0, w0, ac);
@@ -1895,21 +1876,21 @@ __global__ void __launch_bounds__(RowNet<W>::NT, 4) conv_rows_kernel(NetArgs a, 
   }
 }
 
-template <int W, bool FIELDS>
+template <int W>
 int launch_rows(const NetArgs& a, int S, hipStream_t s) {
   using P = RowNet<W>;
   constexpr int lds = P::lds_bytes();
   static_assert(lds * P::WG_PER_CU <= 160 * 1024, "rings do not fit the LDS");
   static bool attr = false;
   if (!attr) {
-    const hipError_t e = hipFuncSetAttribute((const void*)conv_rows_kernel<W, FIELDS>,
+    const hipError_t e = hipFuncSetAttribute((const void*)conv_rows_kernel<W>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess)
       return ddx::set_error(DDX_ERR_HIP, std::string("conv_rows LDS attribute: ") + hipGetErrorString(e));
     attr = true;
   }
   const int strips = (a.H + S - 1) / S;
-  hipLaunchKernelGGL((conv_rows_kernel<W, FIELDS>), dim3((unsigned)(a.B * strips)), dim3(P::NT), lds, s, a, S, strips);
+  hipLaunchKernelGGL((conv_rows_kernel<W>), dim3((unsigned)(a.B * strips)), dim3(P::NT), lds, s, a, S, strips);
   CL_LAUNCHCHK("conv_rows");
   return 0;
 }
@@ -2140,17 +2121,18 @@ int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
   const long big = (H % 16 == 0 && W % 32 == 0) ? (long)B * (H / 16) * (W / 32) : 0;
   const bool small_ok = H % 8 == 0 && W % 16 == 0;
   if (nl == 5 && hid == 32) {
-    // Row by row where its start and steps (6 us, then 1.4 us each with every
-    // CU busy) take less than the tile kernel's rounds of 256 tiles (26.5 us
-    // each): 256 images 64^2 112 us against 213, 128 images 72 against 107;
-    // for 64 images the two are even (53), below that the tiles win.
-    if (big >= 256 && (W == 32 || W == 64) && !x == !out) {
+    // Row by row, between packed arrays, where its start and steps (6 us, then
+    // 1.4 us each with every CU busy) take less than the tile kernel's rounds
+    // of 256 tiles (26.5 us each): 256 images 64^2 105 us against 184, 128
+    // images 66 against 94; for 64 images the two are even, below that the
+    // tiles win.  From float64 fields a step also waits for its row of inputs
+    // and addends, and holding them a step ahead spills: 128 images 114 us
+    // against 113 on tiles, 96 images 109 against 86, so fields stay there.
+    if (x && out && big >= 256 && (W == 32 || W == 64)) {
       int S = 0;
       const long steps = rows_plan(B, H, W == 64 ? RowNet<64>::WG_PER_CU : RowNet<32>::WG_PER_CU, &S);
-      if (60 + 14 * steps < 265 * ((big + 255) / 256)) {
-        if (W == 64) return x ? launch_rows<64, false>(a, S, s) : launch_rows<64, true>(a, S, s);
-        return x ? launch_rows<32, false>(a, S, s) : launch_rows<32, true>(a, S, s);
-      }
+      if (60 + 14 * steps < 265 * ((big + 255) / 256))
+        return W == 64 ? launch_rows<64>(a, S, s) : launch_rows<32>(a, S, s);
     }
     if (big >= 256 || (big > 0 && !small_ok)) return launch_net<5, 32, 32, 16, 768>(a, s);
     // a few images: small tiles, whose layers are a few short dependent

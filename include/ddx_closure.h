@@ -120,8 +120,8 @@ int ddx_box_filter(void* stream, int ny, int nx, int factor, int f64, const void
  * and the layer-by-layer calls apply.  The tile size follows the image
  * count: 32 x 16 output tiles when they alone fill the chip, 4 x 4 when at
  * most 256 of them cover the images (one 64^2 coarse run), 8 x 8 for a few
- * images, 16 x 8 in between; many images 32 or 64 pixels wide (depth 5) run
- * row by row instead, with the same values.  in_scale, out_scale, add may be NULL (1, 1,
+ * images, 16 x 8 in between; from x to out, many images 32 or 64 pixels wide
+ * (depth 5) run row by row instead, with the same values.  in_scale, out_scale, add may be NULL (1, 1,
  * nothing). */
 int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
                  const void* const* w, const float* const* bias, const void* x, float* out,

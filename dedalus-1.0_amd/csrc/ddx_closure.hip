@@ -189,22 +189,33 @@ __device__ inline bf16x8 lds8(const uint16_t* p) {
 // owns 64 of them as four 16-pixel fragments.  Blocks loop over tiles (tile c,
 // c + gridDim.x, ...): the weights are staged in LDS once per block, and the
 // next tile's input halo is loaded into registers while the current tile
-// computes.  The first halo and, for the GELU gradient, a tile's
-// pre-activations are requested before anything waits.  A training batch of
-// 32 images 64^2 (one tile per block) takes 12.8 us per 32-channel layer, the
-// larger part of it the 24 MB of fp32 and bf16 stores: stored straight from
-// the accumulators, in 64-byte pieces instead of the staging's whole lines,
-// it took 13.8.  TC = 32 multiplies 32 channels in two steps of 16, the sums
-// of conv3x3_kernel.  Pixel stride and weight-row stride CI + 4 (bf16) place the
-// 16 rows of a fragment read in distinct bank pairs.  CI = 32 uses the
-// gfx950 16x16x32 bf16 MFMA, CI = 16 the 16x16x16 one.
+// computes.  A training batch of 32 images 64^2 (one tile per block) takes
+// 10.8 us per 32-channel layer, the larger part of it the 24 MB of fp32 and
+// bf16 stores: stored straight from the accumulators, in 64-byte pieces
+// instead of the staging's whole lines, it took a microsecond more.  TC = 32
+// multiplies 32 channels in two steps of 16, the sums of conv3x3_kernel.
+// Pixel stride and weight-row stride CI + 4 (bf16) place the 16 rows of a
+// fragment read in distinct bank pairs.  CI = 32 uses the gfx950 16x16x32
+// bf16 MFMA, CI = 16 the 16x16x16 one.
 //
 // BF (bf16 output only, no fp32 output or GELU gradient: the inference
 // pass): bias and activation are applied to the accumulators and the
 // results staged as bf16, which halves the staging LDS; the kernel then fits
 // three workgroups per CU instead of two.
-template <int CI, int CO, bool BF, int TC>
-__global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs a, long ntiles) {
+//
+// EX (training): sums of the GELU gradient for the bias, and fp32 outputs of
+// fewer than CO channels.  Decided at run time, the two cost every layer call
+// 2 to 20 registers and up to 14 % (one image 512^2, 32 -> 32 channels, both
+// outputs: 20.0 us, 17.4 without).
+//
+// Order of the first requests: the halo, then the weights; the GELU
+// gradient's pre-activations before the products.  With 32 channels in
+// 64-column tiles those registers are short and the reverse is faster (WFIRST:
+// the same call 18.6 -> 17.4 us), and with BF the tile's address is formed
+// after the products (LATE: the bf16-only call 14.8 -> 13.9 us).
+template <int CI, int CO, bool BF, int TC, bool EX, int MINW>
+__global__ void __launch_bounds__(256, MINW) conv3x3_tile_kernel(ConvArgs a, long ntiles) {
+  constexpr bool WFIRST = CI == 32 && TC == 64 && !BF, LATE = CI == 32 && TC == 64 && BF;
   constexpr int PS = CI + 4, WS = CI + 4;
   constexpr int TR = 256 / TC, HR = TR + 2, HC = TC + 2;
   constexpr int NCO = CO / 16;
@@ -255,7 +266,7 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
     for (int j = 0; j < NCO; ++j) biasj[j] = a.bias[j * 16 + m];
   }
   long tile = blockIdx.x;
-  if (tile < ntiles) fetch(tile);
+  if (!WFIRST && tile < ntiles) fetch(tile);
   uint4 wv[WPT];
 #pragma unroll
   for (int k = 0; k < WPT; ++k) {
@@ -272,7 +283,8 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
       d[1] = make_uint2(wv[k].z, wv[k].w);
     }
   }
-  double bsum[4] = {0.0, 0.0, 0.0, 0.0};   // this thread's channels (lane % (CO/4)) * 4 + e over its pixels
+  if (WFIRST && tile < ntiles) fetch(tile);
+  double bsum[4] = {0.0, 0.0, 0.0, 0.0};   // EX: this thread's channels (lane % (CO/4)) * 4 + e over its pixels
   // pixel px of the wavefront's 64: tile row and column
   auto prow = [&](int px) { return TC == 64 ? wave : 2 * wave + (px >> 5); };
   auto pcol = [&](int px) { return TC == 64 ? px : px & 31; };
@@ -291,23 +303,27 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
     lds_barrier();
     const long next = tile + gridDim.x;
     if (next < ntiles) fetch(next);  // in flight while this tile computes
-    long rest = tile;
-    const int tx = (int)(rest % tiles_x);
-    rest /= tiles_x;
-    const int ty = (int)(rest % tiles_y);
-    const int b = (int)(rest / tiles_y);
-    // first pixel of the tile row r
-    const long p00 = ((long)b * a.H + ty * TR) * a.W + tx * TC;
+    long p00 = 0;   // the tile's first pixel
+    auto origin = [&]() {
+      long rest = tile;
+      const int tx = (int)(rest % tiles_x);
+      rest /= tiles_x;
+      const int ty = (int)(rest % tiles_y);
+      const int b = (int)(rest / tiles_y);
+      p00 = ((long)b * a.H + ty * TR) * a.W + tx * TC;
+    };
+    if (!LATE) origin();
     auto gpix = [&](int px) { return p00 + (long)prow(px) * a.W + pcol(px); };
     // pre-activations of this thread's output chunks (see the staging below)
     constexpr int C4 = CO / 4, NR = C4;
     const int c = (lane % C4) * 4;
     float4 zaux[NR];
-    if (!BF && grad) {
+    auto load_aux = [&]() {
 #pragma unroll
       for (int r = 0; r < NR; ++r)
         zaux[r] = *reinterpret_cast<const float4*>(&a.aux[gpix((lane + 64 * r) / C4) * CO + c]);
-    }
+    };
+    if (!BF && !WFIRST && grad) load_aux();
     f32x4 acc[4][NCO];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -346,6 +362,7 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
         }
       }
     }
+    if (LATE) origin();
     lds_barrier();  // every wavefront is done with the halo
     if constexpr (BF) {
       // activations of the D fragments (pixel q*16 + 4kq + i, channel j*16 + m)
@@ -378,6 +395,7 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
 #pragma unroll
         for (int i = 0; i < 4; ++i) st[(q * 16 + 4 * kq + i) * ES + j * 16 + m] = acc[q][j][i];
     lds_barrier();
+    if (WFIRST && grad) load_aux();
     // 4 channels per chunk; a lane's channels c..c+3 are the same in every
     // chunk (C4 divides 64), so its bias was read once before the tile loop
 #pragma unroll
@@ -392,7 +410,7 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
         for (int e = 0; e < 4; ++e) {
           v[e] *= gelu_grad(zz[e]);
           act[e] = v[e];
-          bsum[e] += (double)v[e];
+          if (EX) bsum[e] += (double)v[e];
         }
       } else {
 #pragma unroll
@@ -402,7 +420,7 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
         }
       }
       if (a.out_f32) {
-        if (a.cout == CO) {
+        if (!EX || a.cout == CO) {
           *reinterpret_cast<float4*>(&a.out_f32[o]) = make_float4(v[0], v[1], v[2], v[3]);
         } else {
 #pragma unroll
@@ -416,7 +434,7 @@ __global__ void __launch_bounds__(256, BF ? 3 : 2) conv3x3_tile_kernel(ConvArgs 
                        (uint32_t)f2bf(act[2]) | ((uint32_t)f2bf(act[3]) << 16));
     }
   }
-  if constexpr (!BF) {
+  if constexpr (EX) {
     if (a.bpart) {
       // lanes, then wavefronts, in a fixed order
 #pragma unroll
@@ -950,22 +968,43 @@ int tile_cols(int H, int W, int Ci, int Co) {
 // blocks loop over tiles; about four resident blocks per CU cover the chip
 inline long conv_blocks(long ntiles) { return ntiles < 1024 ? ntiles : 1024; }
 
-template <int CI, int CO, bool BF>
+template <int CI, int CO, bool BF, bool EX>
 void conv_tile_go(hipStream_t s, const ConvArgs& a, int tc) {
   const long ntiles = (long)a.B * a.H * a.W / 256;
   const dim3 grid((unsigned)conv_blocks(ntiles));
-  if (tc == 64) hipLaunchKernelGGL((conv3x3_tile_kernel<CI, CO, BF, 64>), grid, dim3(256), 0, s, a, ntiles);
-  else hipLaunchKernelGGL((conv3x3_tile_kernel<CI, CO, BF, 32>), grid, dim3(256), 0, s, a, ntiles);
+  constexpr int MINW = BF ? 3 : 2;
+  if (tc != 64) {
+    hipLaunchKernelGGL((conv3x3_tile_kernel<CI, CO, BF, 32, EX, MINW>), grid, dim3(256), 0, s, a, ntiles);
+    return;
+  }
+  if constexpr (BF && CI == 32 && CO == 16) {
+    // Up to two workgroups per CU the time is one tile's latency, and the
+    // code for three wavefronts per SIMD reads its operands later: 8 images
+    // 64^2 5.1 us without that bound, 5.6 with it; one image 512^2 (four
+    // workgroups per CU) 10.3 and 9.4.
+    if (ntiles <= 512) {
+      hipLaunchKernelGGL((conv3x3_tile_kernel<CI, CO, BF, 64, EX, 1>), grid, dim3(256), 0, s, a, ntiles);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((conv3x3_tile_kernel<CI, CO, BF, 64, EX, MINW>), grid, dim3(256), 0, s, a, ntiles);
+}
+
+template <bool BF, bool EX>
+void conv_tile_ch(hipStream_t s, const ConvArgs& a, int tc) {
+  switch (a.Ci * 100 + a.Co) {
+    case 1616: conv_tile_go<16, 16, BF, EX>(s, a, tc); break;
+    case 1632: conv_tile_go<16, 32, BF, EX>(s, a, tc); break;
+    case 3216: conv_tile_go<32, 16, BF, EX>(s, a, tc); break;
+    default: conv_tile_go<32, 32, BF, EX>(s, a, tc); break;
+  }
 }
 
 template <bool BF>
 void conv_tile(hipStream_t s, const ConvArgs& a, int tc) {
-  switch (a.Ci * 100 + a.Co) {
-    case 1616: conv_tile_go<16, 16, BF>(s, a, tc); break;
-    case 1632: conv_tile_go<16, 32, BF>(s, a, tc); break;
-    case 3216: conv_tile_go<32, 16, BF>(s, a, tc); break;
-    default: conv_tile_go<32, 32, BF>(s, a, tc); break;
-  }
+  if constexpr (BF) conv_tile_ch<true, false>(s, a, tc);
+  else if (a.bpart || a.cout != a.Co) conv_tile_ch<false, true>(s, a, tc);
+  else conv_tile_ch<false, false>(s, a, tc);
 }
 
 // ddx_conv3x3 with out_f32 holding cout <= Co channels per pixel

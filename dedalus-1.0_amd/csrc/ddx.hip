@@ -609,7 +609,7 @@ int launch_row(ddx_plan* p, RowArgs<T>& a) {
   if (a.mode != ROW_PHYS && p->mix_x && (size_t)2 * a.nx * sizeof(cpx<T>) <= 65536) {
     // plain fields run one per grid row, whatever their number
     ProfScope prof(p, cat, bytes);
-    if (mix_row_launch<T>(p->stream, a, p->mx, nrows)) {
+    if (mix_row_launch<T>(p->stream, a, p->mx, nrows, p->ndim == 2 ? p->ay.n : nrows)) {
       LAUNCHCHK();
       return 0;
     }
@@ -630,7 +630,7 @@ int launch_row(ddx_plan* p, RowArgs<T>& a) {
   }
   if (lds > 65536) return fail(DDX_ERR_UNSUPPORTED, "x rows too long for LDS");
   ProfScope prof(p, cat, bytes);
-  if (!(p->mix_x && mix_row_launch<T>(p->stream, a, p->mx, nrows)))
+  if (!(p->mix_x && mix_row_launch<T>(p->stream, a, p->mx, nrows, nrows)))
     hipLaunchKernelGGL((row_kernel<T>), dim3(nrows), dim3(256), lds, p->stream, a);
   LAUNCHCHK();
   return 0;

@@ -63,7 +63,9 @@ template <typename T> struct RowArgs;
 template <typename T>
 bool mix_col_launch(hipStream_t s, ColArgs<T>& a, const MixPlan& mp, int nslabs, int nfields, int dir,
                     bool spectral);
+// group: rows of which only those of one group may share a transform (the
+// members of a batched plan), nrows if all may; it divides nrows.
 template <typename T>
-bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, long nrows);
+bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, long nrows, long group);
 
 }  // namespace ddx

@@ -569,14 +569,28 @@ mix_row_phys(const RowArgs<T> a, const MixRow mr, long nrows) {
 }
 
 // Plain x-row transforms of one field (blockIdx.y): sequences are row pairs.
+// bpg > 0: every bpg workgroups take a group of nrows rows of its own (a
+// member of a batched plan with an odd number of rows, whose last row would
+// share a transform with the next member's first: an overflow there would
+// reach every row of that member).
+__device__ __forceinline__ long mixr_group(int bpg, long nrows, long& blk) {
+  blk = blockIdx.x;
+  if (bpg <= 0) return 0;
+  const long g = blockIdx.x / (unsigned)bpg;
+  blk -= g * bpg;
+  return g * nrows;
+}
+
 template <typename T, int RL>
-__global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const MixRow mr, long nrows) {
+__global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const MixRow mr, long nrows, int bpg) {
   extern __shared__ __align__(16) unsigned char mix_smem[];
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(mix_smem);
   const cpx<T>* __restrict__ tw = a.tw;
-  const long p0 = (long)blockIdx.x * mr.rows;   // row pairs
+  long blk;
+  const long first = mixr_group(bpg, nrows, blk);
+  const long p0 = blk * mr.rows;   // row pairs
   const int f = blockIdx.y;
-  const cpx<T>* __restrict__ in = a.in[f];
+  const cpx<T>* __restrict__ in = a.in[f] + first * a.kxp;
   auto src = [&](int q, unsigned& oa, unsigned& ob, bool& hasb) {
     const long row = 2 * (p0 + q);
     hasb = row + 1 < nrows;
@@ -593,7 +607,7 @@ __global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const 
 #undef MIX_CALL
     __syncthreads();
   }
-  T* __restrict__ x = a.xout[f];
+  T* __restrict__ x = a.xout[f] + first * mr.n;
   for (int idx = threadIdx.x; idx < mr.rows * mr.T3; idx += blockDim.x) {
     const int rl = mix_div(idx, mr.dT3), t = idx - rl * mr.T3;
     const int k1 = mix_div(t, mr.dR0), k0 = t - k1 * mr.R0;
@@ -615,13 +629,15 @@ __global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const 
 }
 
 template <typename T, int RL>
-__global__ void __launch_bounds__(256) mix_row_r2c(const RowArgs<T> a, const MixRow mr, long nrows) {
+__global__ void __launch_bounds__(256) mix_row_r2c(const RowArgs<T> a, const MixRow mr, long nrows, int bpg) {
   extern __shared__ __align__(16) unsigned char mix_smem[];
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(mix_smem);
   const cpx<T>* __restrict__ tw = a.tw;
-  const long p0 = (long)blockIdx.x * mr.rows;
+  long blk;
+  const long first = mixr_group(bpg, nrows, blk);
+  const long p0 = blk * mr.rows;
   const int f = blockIdx.y;
-  const T* __restrict__ x = a.xin[f];
+  const T* __restrict__ x = a.xin[f] + first * mr.n;
   for (int idx = threadIdx.x; idx < mr.rows * mr.T3; idx += blockDim.x) {
     const int rl = mix_div(idx, mr.dT3), t = idx - rl * mr.T3;
     const int k1 = mix_div(t, mr.dR0), k0 = t - k1 * mr.R0;
@@ -651,7 +667,7 @@ __global__ void __launch_bounds__(256) mix_row_r2c(const RowArgs<T> a, const Mix
   MIX_RADIX10(mr.R0, MIX_CALL)
 #undef MIX_CALL
   __syncthreads();
-  cpx<T>* __restrict__ out = a.out[f];
+  cpx<T>* __restrict__ out = a.out[f] + first * a.kxp;
   for (int idx = threadIdx.x; idx < mr.rows * a.kxp; idx += blockDim.x) {
     const int rl = idx / a.kxp, k = idx - rl * a.kxp;
     const long row = 2 * (p0 + rl);

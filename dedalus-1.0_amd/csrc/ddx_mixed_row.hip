@@ -31,11 +31,13 @@ DDX_MIX_INST(PH_MHD)
 #else
 
 template <typename T>
-bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long nrows) {
+bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long nrows, long group) {
   MixRow mr = mr0;
   const bool phys = a.mode == ROW_PHYS;
   const int nseq = phys ? (a.nin + 1) / 2 : 1;
-  const long units = phys ? nrows : (nrows + 1) / 2;      // rows, or pairs of rows
+  if (phys || group % 2 == 0) group = nrows;              // pairs stay inside the groups by themselves
+  const long upg = phys ? nrows : (group + 1) / 2;        // rows, or pairs of rows of a group
+  const long units = nrows / group * upg;
   const int nf = phys ? 1 : (a.mode == ROW_C2R ? a.nin : a.nout);
   if (phys) {
     // the fields of a right-hand side are equally spaced arrays of one buffer
@@ -54,13 +56,16 @@ bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long 
   // Rows per workgroup: about 256 butterflies per pass within 40 KB of LDS
   // (four workgroups per CU), fewer while CUs would stay without one.
   int rows = 1;
-  while (rows < 8 && 2 * rows * mr.T3 <= 256 && 2 * rows * per <= 40960 && (units / (2 * rows)) * nf >= 512) rows *= 2;
+  while (rows < 8 && 2 * rows <= upg && 2 * rows * mr.T3 <= 256 && 2 * rows * per <= 40960 &&
+         (units / (2 * rows)) * nf >= 512)
+    rows *= 2;
   mr.rows = rows;
   int thr = rows * (mr.T3 > nseq * mr.J ? mr.T3 : nseq * mr.J);
   thr = (thr + 63) / 64 * 64;
   if (thr > 256) thr = 256;
   const size_t lds = rows * per;
-  const unsigned blocks = (unsigned)((units + rows - 1) / rows);
+  const unsigned bpg = (unsigned)((upg + rows - 1) / rows);
+  const unsigned blocks = bpg * (unsigned)(nrows / group);
   if (phys) {
     switch (a.physics * 10 + a.ndim) {
       case PH_HYDRO * 10 + 2: mix_row_phys_go<T, PH_HYDRO, 2>(s, a, mr, blocks, thr, lds, nrows); break;
@@ -74,20 +79,21 @@ bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long 
     return true;
   }
   const dim3 grid(blocks, (unsigned)nf);
+  const int gb = group < nrows ? (int)bpg : 0;
   if (a.mode == ROW_C2R) {
-    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_c2r<T, 4>), grid, dim3(thr), lds, s, a, mr, nrows);
-    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_c2r<T, 5>), grid, dim3(thr), lds, s, a, mr, nrows);
-    else hipLaunchKernelGGL((mix_row_c2r<T, 6>), grid, dim3(thr), lds, s, a, mr, nrows);
+    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_c2r<T, 4>), grid, dim3(thr), lds, s, a, mr, group, gb);
+    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_c2r<T, 5>), grid, dim3(thr), lds, s, a, mr, group, gb);
+    else hipLaunchKernelGGL((mix_row_c2r<T, 6>), grid, dim3(thr), lds, s, a, mr, group, gb);
   } else {
-    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_r2c<T, 4>), grid, dim3(thr), lds, s, a, mr, nrows);
-    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_r2c<T, 5>), grid, dim3(thr), lds, s, a, mr, nrows);
-    else hipLaunchKernelGGL((mix_row_r2c<T, 6>), grid, dim3(thr), lds, s, a, mr, nrows);
+    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_r2c<T, 4>), grid, dim3(thr), lds, s, a, mr, group, gb);
+    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_r2c<T, 5>), grid, dim3(thr), lds, s, a, mr, group, gb);
+    else hipLaunchKernelGGL((mix_row_r2c<T, 6>), grid, dim3(thr), lds, s, a, mr, group, gb);
   }
   return true;
 }
 
-template bool mix_row_launch<double>(hipStream_t, const RowArgs<double>&, const MixRow&, long);
-template bool mix_row_launch<float>(hipStream_t, const RowArgs<float>&, const MixRow&, long);
+template bool mix_row_launch<double>(hipStream_t, const RowArgs<double>&, const MixRow&, long, long);
+template bool mix_row_launch<float>(hipStream_t, const RowArgs<float>&, const MixRow&, long, long);
 
 #endif
 

@@ -172,6 +172,19 @@ __device__ inline void row_physics(int physics, int ndim, T fi, const T* q, T* o
   }
 }
 
+// First row of the group, and workgroup in it, of a plain row transform,
+// which takes rows in pairs.  bpg > 0: every bpg workgroups take a group of
+// nrows rows of its own (a member of a batched plan with an odd number of
+// rows, whose last row would share a transform with the next member's first:
+// an overflow there would reach every row of that member).
+__device__ __forceinline__ long row_group(int bpg, long nrows, long& blk) {
+  blk = blockIdx.x;
+  if (bpg <= 0) return 0;
+  const long g = blockIdx.x / (unsigned)bpg;
+  blk -= g * bpg;
+  return g * nrows;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) row_kernel(const RowArgs<T> a) {
   extern __shared__ unsigned char smem_raw[];

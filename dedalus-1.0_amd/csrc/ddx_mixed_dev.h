@@ -568,18 +568,8 @@ mix_row_phys(const RowArgs<T> a, const MixRow mr, long nrows) {
   }
 }
 
-// Plain x-row transforms of one field (blockIdx.y): sequences are row pairs.
-// bpg > 0: every bpg workgroups take a group of nrows rows of its own (a
-// member of a batched plan with an odd number of rows, whose last row would
-// share a transform with the next member's first: an overflow there would
-// reach every row of that member).
-__device__ __forceinline__ long mixr_group(int bpg, long nrows, long& blk) {
-  blk = blockIdx.x;
-  if (bpg <= 0) return 0;
-  const long g = blockIdx.x / (unsigned)bpg;
-  blk -= g * bpg;
-  return g * nrows;
-}
+// Plain x-row transforms of one field (blockIdx.y): sequences are row pairs
+// (of one group each, row_group).
 
 template <typename T, int RL>
 __global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const MixRow mr, long nrows, int bpg) {
@@ -587,7 +577,7 @@ __global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const 
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(mix_smem);
   const cpx<T>* __restrict__ tw = a.tw;
   long blk;
-  const long first = mixr_group(bpg, nrows, blk);
+  const long first = row_group(bpg, nrows, blk);
   const long p0 = blk * mr.rows;   // row pairs
   const int f = blockIdx.y;
   const cpx<T>* __restrict__ in = a.in[f] + first * a.kxp;
@@ -634,7 +624,7 @@ __global__ void __launch_bounds__(256) mix_row_r2c(const RowArgs<T> a, const Mix
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(mix_smem);
   const cpx<T>* __restrict__ tw = a.tw;
   long blk;
-  const long first = mixr_group(bpg, nrows, blk);
+  const long first = row_group(bpg, nrows, blk);
   const long p0 = blk * mr.rows;
   const int f = blockIdx.y;
   const T* __restrict__ x = a.xin[f] + first * mr.n;

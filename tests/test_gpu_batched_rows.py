@@ -15,11 +15,12 @@ pytestmark = pytest.mark.gpu
 
 
 # mixed-radix rows with one, two and eight row pairs to a workgroup, a row
-# count that leaves most of a workgroup empty, the general row kernel (576)
-# and an even row count
+# count that leaves most of a workgroup empty, the general row kernel (576),
+# an even row count, and the size-specialised rows
 @pytest.mark.parametrize("f32", [False, True], ids=["f64", "f32"])
 @pytest.mark.parametrize("batch,shape", [(3, (5, 20)), (33, (75, 90)), (301, (45, 30)), (700, (3, 40)), (64, (15, 360)),
-                                         (2, (9, 576)), (8, (48, 48)), (1, (9, 20))], ids=str)
+                                         (2, (9, 576)), (8, (48, 48)), (5, (75, 64)), (90, (9, 128)), (3, (27, 256)),
+                                         (40, (45, 512)), (1, (9, 64))], ids=str)
 def test_members_are_independent(batch, shape, f32):
     hp = hip()
     case("batched rows", batch, shape, f32)

@@ -1934,18 +1934,46 @@ int launch_rows(const NetArgs& a, int S, hipStream_t s) {
   return 0;
 }
 
-// Strip height of the row kernel for B images of H rows, and the rounds of
-// steps it takes: the strips run in rounds of 256 CUs' workgroups, a strip of
-// S rows takes S + 17 steps.
-long rows_plan(int B, int H, int per_cu, int* S) {
+// Strip height of the row kernel for B images of H rows: the strips run in
+// rounds of 256 CUs' workgroups, a strip of S rows takes S + 17 steps.
+int rows_plan(int B, int H, int per_cu) {
   long best = -1;
+  int S = H;
   for (int n = 1; n <= 8 && n <= H; ++n) {
     const int s = (H + n - 1) / n;
     const long wgs = (long)B * ((H + s - 1) / s);
     const long cost = ((wgs + 256L * per_cu - 1) / (256L * per_cu)) * (s + 17);
-    if (best < 0 || cost < best) { best = cost; *S = s; }
+    if (best < 0 || cost < best) { best = cost; S = s; }
   }
-  return best;
+  return S;
+}
+
+// Strip height where the network of depth 5 and width 32 runs row by row
+// between packed arrays, 0 where it runs on tiles.  Both kernels' times are
+// sums of rounds, fitted (in ns) to 292 shapes of 256 to 4096 tiles, 16 to 512
+// rows (nine in ten within 5 %; a few strips 32 wide run faster than the
+// sum): the tiles take 22.2 us for every 256, a 64-wide strip 6.6
+// us to start and 1.15 a step.  Of the 32-wide ones two share a CU: a step
+// takes 0.83 us alone, 1.26 where every CU holds two.  256 images 64^2 105 us
+// against 184, 128 images 66 against 94; 64 images are even (47.4 and 47.0).
+// Short strips in several rounds lose to the tiles: 1150 images 16 x 64 220 us
+// against 203, 128 images 64 x 32 48.5 against 46.3.
+// From float64 fields a step also waits for its row of inputs and addends,
+// and holding them a step ahead spills: 128 images 114 us against 113 on
+// tiles, 96 images 109 against 86, so fields stay on tiles.
+int rows_strip(int B, int H, int W, int nl, int hid) {
+  const long big = (H % 16 == 0 && W % 32 == 0) ? (long)B * (H / 16) * (W / 32) : 0;
+  if (nl != 5 || hid != 32 || big < 256 || (W != 32 && W != 64)) return 0;
+  const int S = rows_plan(B, H, W == 64 ? RowNet<64>::WG_PER_CU : RowNet<32>::WG_PER_CU);
+  const long wgs = (long)B * ((H + S - 1) / S), steps = S + 17;
+  long ns;
+  if (W == 64) {
+    ns = 1000 + ((wgs + 255) / 256) * (6600 + 1150 * steps);
+  } else {
+    const long full = wgs / 512, rest = wgs % 512;
+    ns = 6000 + steps * (1260 * full + (rest == 0 ? 0 : rest <= 256 ? 830 : 830 + 460 * rest / 512));
+  }
+  return ns < 3000 + 22200 * ((big + 255) / 256) ? S : 0;
 }
 
 }  // namespace
@@ -2160,18 +2188,9 @@ int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
   const long big = (H % 16 == 0 && W % 32 == 0) ? (long)B * (H / 16) * (W / 32) : 0;
   const bool small_ok = H % 8 == 0 && W % 16 == 0;
   if (nl == 5 && hid == 32) {
-    // Row by row, between packed arrays, where its start and steps (6 us, then
-    // 1.4 us each with every CU busy) take less than the tile kernel's rounds
-    // of 256 tiles (26.5 us each): 256 images 64^2 105 us against 184, 128
-    // images 66 against 94; for 64 images the two are even, below that the
-    // tiles win.  From float64 fields a step also waits for its row of inputs
-    // and addends, and holding them a step ahead spills: 128 images 114 us
-    // against 113 on tiles, 96 images 109 against 86, so fields stay there.
-    if (x && out && big >= 256 && (W == 32 || W == 64)) {
-      int S = 0;
-      const long steps = rows_plan(B, H, W == 64 ? RowNet<64>::WG_PER_CU : RowNet<32>::WG_PER_CU, &S);
-      if (60 + 14 * steps < 265 * ((big + 255) / 256))
-        return W == 64 ? launch_rows<64>(a, S, s) : launch_rows<32>(a, S, s);
+    if (x && out) {
+      const int S = rows_strip(B, H, W, nl, hid);
+      if (S) return W == 64 ? launch_rows<64>(a, S, s) : launch_rows<32>(a, S, s);
     }
     if (big >= 256 || (big > 0 && !small_ok)) return launch_net<5, 32, 32, 16, 768>(a, s);
     // a few images: small tiles, whose layers are a few short dependent
@@ -2194,6 +2213,13 @@ int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
   return ddx::set_error(DDX_ERR_UNSUPPORTED,
                         "fused network: depth 5 width 32 on images of multiples of 8 x 8 "
                         "pixels, or depth 3 width 16 on multiples of 8 x 16");
+}
+
+int ddx_conv_net_rows(int B, int H, int W, int nl, const int* chans) {
+  if (B < 1 || H < 1 || W < 1 || nl < 2 || nl > NET_MAXL || !chans) return 0;
+  for (int l = 2; l < nl; ++l)
+    if (chans[l] != chans[1]) return 0;
+  return rows_strip(B, H, W, nl, chans[1]);
 }
 
 int ddx_net_bytes(int B, int H, int W, int nl, const int* chans, int64_t* saved, int64_t* scratch) {

@@ -118,6 +118,7 @@ SIGNATURES = {
     "ddx_conv_pack": (_I, [_VP, ctypes.c_int64, _I, _I, _PP, ctypes.c_int64, _I, _VP, _VP, _VP]),
     "ddx_conv_unpack": (_I, [_VP, ctypes.c_int64, _I, _I, _VP, _PP, ctypes.c_int64, _I, _VP, _PP]),
     "ddx_box_filter": (_I, [_VP, _I, _I, _I, _I, _VP, _VP]),
+    "ddx_conv_net_rows": (_I, [_I, _I, _I, _I, ctypes.POINTER(_I)]),
     "ddx_net_bytes": (_I, [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(ctypes.c_int64),
                            ctypes.POINTER(ctypes.c_int64)]),
     "ddx_net_forward": (_I, [_VP, _I, _I, _I, _I, ctypes.POINTER(_I), _VP, _PP, _PP, _VP, _VP]),

@@ -128,6 +128,10 @@ int ddx_conv_net(void* stream, int B, int H, int W, int nl, const int* chans,
                  const void* const* src, const float* in_scale, void* const* dst,
                  const void* const* add, const float* out_scale);
 
+/* Rows per strip where ddx_conv_net from x to out runs row by row, 0 where it
+ * runs on tiles (host only, no device needed). */
+int ddx_conv_net_rows(int B, int H, int W, int nl, const int* chans);
+
 /* Training.  The network of ddx_conv_net's description with any depth and
  * widths ddx_conv3x3 takes (inputs of at most 16 channels): ddx_net_forward
  * gives out [npix][chans[nl]] fp32 from x [npix][chans[0]] fp32 and the fp32

@@ -38,3 +38,44 @@ def test_rows_match_layers(B, H, W):
     unpack(ref.run(), 2, p(want), True, scale=[0.3, 0.4], add=p(add))
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def same(a, b):
+    """Bit for bit, NaN for NaN."""
+    return bool(((a == b) | (a.isnan() & b.isnan())).all())
+
+
+# as the rule has it (asserted): one strip per image, several, a shorter last
+# strip, 16-row images in one round and in two, 32-wide images alone on a CU
+# and two to a CU; values that overflow, NaN, and products below the normal range
+@pytest.mark.parametrize("values", ["normal", "tiny", "nonfinite"])
+@pytest.mark.parametrize("B,H,W,S", [(256, 64, 64, 64), (128, 64, 64, 32), (67, 48, 64, 16), (40, 80, 64, 14),
+                                     (400, 16, 64, 16), (200, 16, 64, 16), (25, 512, 32, 64), (19, 256, 32, 32),
+                                     (300, 16, 32, 16), (600, 64, 32, 32), (1024, 32, 32, 32)])
+def test_row_kernel(B, H, W, S, values):
+    import ctypes
+    from dedalus import _hip
+    from dedalus.closure.net import ClosureNet, Inference
+    _hip.init()
+    chans = (3, 32, 32, 32, 32, 2)
+    assert _hip._lib.ddx_conv_net_rows(B, H, W, 5, (ctypes.c_int * 6)(*chans)) == S
+    print("case: row kernel", B, H, W, values, flush=True)
+    torch.manual_seed(B + H + W)
+    net = ClosureNet(cin=3, cout=2, width=32, depth=5, seed=2, out_scale=1.0).cuda()
+    with torch.no_grad():
+        for b in net.biases:
+            b.normal_(0, 1e-38 if values == "tiny" else 0.1)
+    one, ref = Inference(net, B, H, W), Inference(net, B, H, W, fused=False)
+    x = torch.randn(B * H * W, 3, device="cuda")
+    if values == "tiny":
+        x *= 1e-37
+    elif values == "nonfinite":
+        x[W // 2] = float("inf")                   # first row of the first image
+        x[(B - 1) * H * W + H * W // 2] = float("nan")
+        x[(B // 2) * H * W + 3] = 3e38
+    one.x[:, :3] = x.bfloat16()
+    ref.x.copy_(one.x)
+    got, want = one.run(), ref.run()
+    assert same(got, want)
+    if values == "nonfinite" and B > 4:
+        assert got.view(B, -1)[1].isfinite().all()

@@ -556,14 +556,13 @@ bool launch_row_fast(ddx_plan* p, const RowArgs<T>& a, long nrows) {
 template <typename T, int N, int V>
 void row_plain_nv(ddx_plan* p, const RowArgs<T>& a, long nrows) {
   constexpr int RPB = 64 / RowPlanV<N, V>::LANES;
-  // an odd number of rows per member: groups of workgroups per member
-  const long group = p->ndim == 2 && p->ay.n % 2 ? p->ay.n : nrows;
-  const long teams = (group + 1) / 2, bpg = (teams + RPB - 1) / RPB;
-  const int gb = group < nrows ? (int)bpg : 0;
+  // members of an odd number of rows pair their rows inside the member
+  const int group = p->ndim == 2 && p->nbatch > 1 && p->ay.n % 2 ? p->ay.n : 0;
+  const long teams = group ? nrows / group * ((group + 1) / 2) : (nrows + 1) / 2;
   const int nf = a.mode == ROW_C2R ? a.nin : a.nout;   // grid.y: the field
-  const dim3 grid((unsigned)(bpg * (nrows / group)), (unsigned)nf);
-  if (a.mode == ROW_C2R) hipLaunchKernelGGL((row_c2r_fast<T, N, V>), grid, dim3(64), 0, p->stream, a, group, gb);
-  else hipLaunchKernelGGL((row_r2c_fast<T, N, V>), grid, dim3(64), 0, p->stream, a, group, gb);
+  const dim3 grid((unsigned)((teams + RPB - 1) / RPB), (unsigned)nf);
+  if (a.mode == ROW_C2R) hipLaunchKernelGGL((row_c2r_fast<T, N, V>), grid, dim3(64), 0, p->stream, a, nrows, group);
+  else hipLaunchKernelGGL((row_r2c_fast<T, N, V>), grid, dim3(64), 0, p->stream, a, nrows, group);
 }
 
 template <typename T, int N>

@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(64) row_phys_fast(const RowArgs<T> a, long nro
 // inverse transform, x rows = (Re z, Im z).  Loads as in row_phys_fast
 // (clamped addresses, zeroed afterwards, the k = 0 imaginary part dropped).
 template <typename T, int N, int V = 0>
-__global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrows, int bpg) {
+__global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrows, int group) {
   using PL = RowPlanV<N, V>;
   constexpr int LANES = PL::LANES, E = PL::E, RPB = 64 / LANES;
   constexpr int R0 = PL::R[0], RL = PL::R[PL::NP - 1];
@@ -515,17 +515,16 @@ __global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrow
   constexpr bool POW = sizeof(T) == 8;
   __shared__ cpx<T> lds[RPB][BUF];
   const int team = threadIdx.x / LANES, lane = threadIdx.x % LANES;
-  long blk;
-  const long first = row_group(bpg, nrows, blk);
-  const long ra = 2 * (blk * RPB + team), rb = ra + 1;
-  const bool live_a = ra < nrows, live_b = rb < nrows;
-  const long la_row = live_a ? ra : nrows - 1, lb_row = live_b ? rb : nrows - 1;
+  long ra;
+  bool live_a, live_b;
+  row_pair((long)blockIdx.x * RPB + team, nrows, group, ra, live_a, live_b);
+  const long la_row = live_a ? ra : nrows - 1, lb_row = live_b ? ra + 1 : nrows - 1;
   const int cx = a.kx - 1;
   cpx<T> twc[PL::NP][E];
   fill_twiddles<T, N, PL, false, POW>(twc, lane, a.tw);
   const int f = blockIdx.y;   // the field
-  const cpx<T>* __restrict__ ia = a.in[f] + (first + la_row) * a.kxp;
-  const cpx<T>* __restrict__ ib = a.in[f] + (first + lb_row) * a.kxp;
+  const cpx<T>* __restrict__ ia = a.in[f] + la_row * a.kxp;
+  const cpx<T>* __restrict__ ib = a.in[f] + lb_row * a.kxp;
   cpx<T> va[E], vb[E];
 #pragma unroll
   for (int qq = 0; qq < E / R0; ++qq)
@@ -552,7 +551,7 @@ __global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrow
       v[e] = keep ? mk(va[e].x - by, ay + bx) : mk(T(0), T(0));
     }
   run_passes_cached<T, 1, N, PL, false, 1, POW>(v, lane, 0, lds[team], twc);
-  T* __restrict__ xa = a.xout[f] + (first + ra) * (long)N;
+  T* __restrict__ xa = a.xout[f] + ra * (long)N;
 #pragma unroll
   for (int qq = 0; qq < E / RL; ++qq)
 #pragma unroll
@@ -567,7 +566,7 @@ __global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrow
 // spectra A = (Z_k + conj Z_{N-k}) / 2, B = (Z_k - conj Z_{N-k}) / 2i.  The
 // x loads sit at the first-pass positions of the reversed radix order.
 template <typename T, int N, int V = 0>
-__global__ void __launch_bounds__(64) row_r2c_fast(const RowArgs<T> a, long nrows, int bpg) {
+__global__ void __launch_bounds__(64) row_r2c_fast(const RowArgs<T> a, long nrows, int group) {
   using PL = RowPlanV<N, V>;
   constexpr int LANES = PL::LANES, E = PL::E, RPB = 64 / LANES;
   constexpr int RL = PL::R[PL::NP - 1], RF = PL::R[0];
@@ -576,17 +575,16 @@ __global__ void __launch_bounds__(64) row_r2c_fast(const RowArgs<T> a, long nrow
   constexpr bool UNI = uniform_radix<PL>();
   __shared__ cpx<T> lds[RPB][BUF];
   const int team = threadIdx.x / LANES, lane = threadIdx.x % LANES;
-  long blk;
-  const long first = row_group(bpg, nrows, blk);
-  const long ra = 2 * (blk * RPB + team), rb = ra + 1;
-  const bool live_a = ra < nrows, live_b = rb < nrows;
-  const long la_row = live_a ? ra : nrows - 1, lb_row = live_b ? rb : nrows - 1;
+  long ra;
+  bool live_a, live_b;
+  row_pair((long)blockIdx.x * RPB + team, nrows, group, ra, live_a, live_b);
+  const long la_row = live_a ? ra : nrows - 1, lb_row = live_b ? ra + 1 : nrows - 1;
   cpx<T>* buf = lds[team];
   cpx<T> twf[PL::NP][E];
   fill_twiddles<T, N, PL, true, POW>(twf, lane, a.tw);
   const int f = blockIdx.y;   // the field
-  const T* __restrict__ xa = a.xin[f] + (first + la_row) * (long)N;
-  const T* __restrict__ xb = a.xin[f] + (first + lb_row) * (long)N;
+  const T* __restrict__ xa = a.xin[f] + la_row * (long)N;
+  const T* __restrict__ xb = a.xin[f] + lb_row * (long)N;
   cpx<T> v[E];
 #pragma unroll
   for (int qq = 0; qq < E / RL; ++qq)
@@ -602,7 +600,7 @@ __global__ void __launch_bounds__(64) row_r2c_fast(const RowArgs<T> a, long nrow
 #pragma unroll
     for (int rr = 0; rr < RF; ++rr) buf[final_pos<N, PL, true>(lane, qq, rr)] = v[qq * RF + rr];
   __syncthreads();
-  cpx<T>* __restrict__ oa = a.out[f] + (first + ra) * (long)a.kxp;
+  cpx<T>* __restrict__ oa = a.out[f] + ra * (long)a.kxp;
   for (int k = lane; k < a.kxp; k += LANES) {
     cpx<T> A = mk(T(0), T(0)), B = mk(T(0), T(0));
     if (k < a.kx) {

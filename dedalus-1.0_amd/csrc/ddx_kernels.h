@@ -172,17 +172,22 @@ __device__ inline void row_physics(int physics, int ndim, T fi, const T* q, T* o
   }
 }
 
-// First row of the group, and workgroup in it, of a plain row transform,
-// which takes rows in pairs.  bpg > 0: every bpg workgroups take a group of
-// nrows rows of its own (a member of a batched plan with an odd number of
-// rows, whose last row would share a transform with the next member's first:
-// an overflow there would reach every row of that member).
-__device__ __forceinline__ long row_group(int bpg, long nrows, long& blk) {
-  blk = blockIdx.x;
-  if (bpg <= 0) return 0;
-  const long g = blockIdx.x / (unsigned)bpg;
-  blk -= g * bpg;
-  return g * nrows;
+// Rows of pair u of a plain row transform: row and, where two is set, row + 1;
+// live is false past the last pair.  group > 0: pairs stay inside groups of
+// that many rows (the members of a batched plan with an odd number of rows,
+// where a member's last row would share a transform with the next member's
+// first: an overflow there would reach every row of that member).
+__device__ __forceinline__ void row_pair(long u, long nrows, int group, long& row, bool& live, bool& two) {
+  if (group <= 0) {
+    row = 2 * u;
+    live = row < nrows;
+    two = row + 1 < nrows;
+  } else {
+    const unsigned per = (unsigned)(group + 1) / 2, g = (unsigned)u / per, j = (unsigned)u - g * per;
+    row = (long)g * group + 2 * j;
+    live = row < nrows;
+    two = live && (int)(2 * j + 1) < group;
+  }
 }
 
 template <typename T>

@@ -569,22 +569,22 @@ mix_row_phys(const RowArgs<T> a, const MixRow mr, long nrows) {
 }
 
 // Plain x-row transforms of one field (blockIdx.y): sequences are row pairs
-// (of one group each, row_group).
+// (row_pair; GRP: within groups, apart because the division it takes costs
+// 2 % of the 3 x 160x144x180 c2r where it is not needed).
 
-template <typename T, int RL>
-__global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const MixRow mr, long nrows, int bpg) {
+template <typename T, int RL, bool GRP>
+__global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const MixRow mr, long nrows, int group) {
   extern __shared__ __align__(16) unsigned char mix_smem[];
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(mix_smem);
   const cpx<T>* __restrict__ tw = a.tw;
-  long blk;
-  const long first = row_group(bpg, nrows, blk);
-  const long p0 = blk * mr.rows;   // row pairs
+  const long p0 = (long)blockIdx.x * mr.rows;   // row pairs
   const int f = blockIdx.y;
-  const cpx<T>* __restrict__ in = a.in[f] + first * a.kxp;
+  const cpx<T>* __restrict__ in = a.in[f];
   auto src = [&](int q, unsigned& oa, unsigned& ob, bool& hasb) {
-    const long row = 2 * (p0 + q);
-    hasb = row + 1 < nrows;
-    oa = (unsigned)(row < nrows ? row : nrows - 1) * (unsigned)a.kxp;
+    long row;
+    bool live;
+    row_pair(p0 + q, nrows, GRP ? group : 0, row, live, hasb);
+    oa = (unsigned)(live ? row : nrows - 1) * (unsigned)a.kxp;
     ob = hasb ? oa + (unsigned)a.kxp : oa;
   };
 #define MIX_CALL(R) mixr_first<T, R>(mr, tw, buf, mr.rows, a.kx - 1, in, src)
@@ -597,7 +597,7 @@ __global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const 
 #undef MIX_CALL
     __syncthreads();
   }
-  T* __restrict__ x = a.xout[f] + first * mr.n;
+  T* __restrict__ x = a.xout[f];
   for (int idx = threadIdx.x; idx < mr.rows * mr.T3; idx += blockDim.x) {
     const int rl = mix_div(idx, mr.dT3), t = idx - rl * mr.T3;
     const int k1 = mix_div(t, mr.dR0), k0 = t - k1 * mr.R0;
@@ -606,10 +606,11 @@ __global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const 
 #pragma unroll
     for (int r = 0; r < RL; ++r) v[r] = b[r * mr.S2];
     mdft<1, RL>(v);
-    const long row = 2 * (p0 + rl);
-    if (row >= nrows) continue;
+    long row;
+    bool live, two;
+    row_pair(p0 + rl, nrows, GRP ? group : 0, row, live, two);
+    if (!live) continue;
     T* xa = x + row * mr.n + t;
-    const bool two = row + 1 < nrows;
 #pragma unroll
     for (int r = 0; r < RL; ++r) {
       xa[r * mr.T3] = v[r].x;
@@ -618,22 +619,21 @@ __global__ void __launch_bounds__(256, 4) mix_row_c2r(const RowArgs<T> a, const 
   }
 }
 
-template <typename T, int RL>
-__global__ void __launch_bounds__(256) mix_row_r2c(const RowArgs<T> a, const MixRow mr, long nrows, int bpg) {
+template <typename T, int RL, bool GRP>
+__global__ void __launch_bounds__(256) mix_row_r2c(const RowArgs<T> a, const MixRow mr, long nrows, int group) {
   extern __shared__ __align__(16) unsigned char mix_smem[];
   cpx<T>* buf = reinterpret_cast<cpx<T>*>(mix_smem);
   const cpx<T>* __restrict__ tw = a.tw;
-  long blk;
-  const long first = row_group(bpg, nrows, blk);
-  const long p0 = blk * mr.rows;
+  const long p0 = (long)blockIdx.x * mr.rows;
   const int f = blockIdx.y;
-  const T* __restrict__ x = a.xin[f] + first * mr.n;
+  const T* __restrict__ x = a.xin[f];
   for (int idx = threadIdx.x; idx < mr.rows * mr.T3; idx += blockDim.x) {
     const int rl = mix_div(idx, mr.dT3), t = idx - rl * mr.T3;
     const int k1 = mix_div(t, mr.dR0), k0 = t - k1 * mr.R0;
-    const long row = 2 * (p0 + rl);
-    const bool two = row + 1 < nrows;
-    const T* xa = x + (row < nrows ? row : nrows - 1) * mr.n + t;
+    long row;
+    bool live, two;
+    row_pair(p0 + rl, nrows, GRP ? group : 0, row, live, two);
+    const T* xa = x + (live ? row : nrows - 1) * mr.n + t;
     const T* xb = x + (two ? row + 1 : nrows - 1) * mr.n + t;
     cpx<T> v[RL];
 #pragma unroll
@@ -657,15 +657,17 @@ __global__ void __launch_bounds__(256) mix_row_r2c(const RowArgs<T> a, const Mix
   MIX_RADIX10(mr.R0, MIX_CALL)
 #undef MIX_CALL
   __syncthreads();
-  cpx<T>* __restrict__ out = a.out[f] + first * a.kxp;
+  cpx<T>* __restrict__ out = a.out[f];
   for (int idx = threadIdx.x; idx < mr.rows * a.kxp; idx += blockDim.x) {
     const int rl = idx / a.kxp, k = idx - rl * a.kxp;
-    const long row = 2 * (p0 + rl);
-    if (row >= nrows) continue;
+    long row;
+    bool live, two;
+    row_pair(p0 + rl, nrows, GRP ? group : 0, row, live, two);
+    if (!live) continue;
     cpx<T> A, B;
     mixr_unpair(mr, buf + rl * mr.SS, k, a.kx, A, B);
     out[row * a.kxp + k] = A;
-    if (row + 1 < nrows) out[(row + 1) * a.kxp + k] = B;
+    if (two) out[(row + 1) * a.kxp + k] = B;
   }
 }
 

@@ -30,14 +30,28 @@ DDX_MIX_INST(PH_MHD)
 
 #else
 
+template <typename T, bool GRP>
+static void mix_row_plain_go(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, dim3 grid, unsigned thr, size_t lds,
+                             long nrows, int group) {
+  if (a.mode == ROW_C2R) {
+    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_c2r<T, 4, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_c2r<T, 5, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else hipLaunchKernelGGL((mix_row_c2r<T, 6, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+  } else {
+    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_r2c<T, 4, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_r2c<T, 5, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else hipLaunchKernelGGL((mix_row_r2c<T, 6, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+  }
+}
+
 template <typename T>
 bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long nrows, long group) {
   MixRow mr = mr0;
   const bool phys = a.mode == ROW_PHYS;
   const int nseq = phys ? (a.nin + 1) / 2 : 1;
-  if (phys || group % 2 == 0) group = nrows;              // pairs stay inside the groups by themselves
-  const long upg = phys ? nrows : (group + 1) / 2;        // rows, or pairs of rows of a group
-  const long units = nrows / group * upg;
+  if (phys || group % 2 == 0 || group >= nrows) group = 0;   // pairs stay inside the groups by themselves
+  // rows, or pairs of rows
+  const long units = phys ? nrows : group ? nrows / group * ((group + 1) / 2) : (nrows + 1) / 2;
   const int nf = phys ? 1 : (a.mode == ROW_C2R ? a.nin : a.nout);
   if (phys) {
     // the fields of a right-hand side are equally spaced arrays of one buffer
@@ -56,16 +70,13 @@ bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long 
   // Rows per workgroup: about 256 butterflies per pass within 40 KB of LDS
   // (four workgroups per CU), fewer while CUs would stay without one.
   int rows = 1;
-  while (rows < 8 && 2 * rows <= upg && 2 * rows * mr.T3 <= 256 && 2 * rows * per <= 40960 &&
-         (units / (2 * rows)) * nf >= 512)
-    rows *= 2;
+  while (rows < 8 && 2 * rows * mr.T3 <= 256 && 2 * rows * per <= 40960 && (units / (2 * rows)) * nf >= 512) rows *= 2;
   mr.rows = rows;
   int thr = rows * (mr.T3 > nseq * mr.J ? mr.T3 : nseq * mr.J);
   thr = (thr + 63) / 64 * 64;
   if (thr > 256) thr = 256;
   const size_t lds = rows * per;
-  const unsigned bpg = (unsigned)((upg + rows - 1) / rows);
-  const unsigned blocks = bpg * (unsigned)(nrows / group);
+  const unsigned blocks = (unsigned)((units + rows - 1) / rows);
   if (phys) {
     switch (a.physics * 10 + a.ndim) {
       case PH_HYDRO * 10 + 2: mix_row_phys_go<T, PH_HYDRO, 2>(s, a, mr, blocks, thr, lds, nrows); break;
@@ -79,16 +90,8 @@ bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long 
     return true;
   }
   const dim3 grid(blocks, (unsigned)nf);
-  const int gb = group < nrows ? (int)bpg : 0;
-  if (a.mode == ROW_C2R) {
-    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_c2r<T, 4>), grid, dim3(thr), lds, s, a, mr, group, gb);
-    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_c2r<T, 5>), grid, dim3(thr), lds, s, a, mr, group, gb);
-    else hipLaunchKernelGGL((mix_row_c2r<T, 6>), grid, dim3(thr), lds, s, a, mr, group, gb);
-  } else {
-    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_r2c<T, 4>), grid, dim3(thr), lds, s, a, mr, group, gb);
-    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_r2c<T, 5>), grid, dim3(thr), lds, s, a, mr, group, gb);
-    else hipLaunchKernelGGL((mix_row_r2c<T, 6>), grid, dim3(thr), lds, s, a, mr, group, gb);
-  }
+  if (group) mix_row_plain_go<T, true>(s, a, mr, grid, thr, lds, nrows, (int)group);
+  else mix_row_plain_go<T, false>(s, a, mr, grid, thr, lds, nrows, 0);
   return true;
 }
 

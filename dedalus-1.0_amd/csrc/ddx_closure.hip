@@ -1993,7 +1993,8 @@ int ddx_conv3x3_wgrad(void* stream, int B, int H, int W, int Ci, int Co, const v
   const long npix = (long)B * H * W;
   hipStream_t s = (hipStream_t)stream;
   const long n = (long)Co * 9 * Ci;
-  const int tc = tile_cols(H, W, Ci, Co);
+  // the tile kernel reads both arrays 8 bytes at a time
+  const int tc = ((uintptr_t)x | (uintptr_t)dz) % 8 == 0 ? tile_cols(H, W, Ci, Co) : 0;
   if (tc) {
     const int nch = wgrad_tiles(s, B, H, W, Ci, Co, tc, x, dz, nullptr, partial, nullptr, nchunk);
     CL_LAUNCHCHK("conv3x3_wgrad tile");

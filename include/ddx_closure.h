@@ -54,7 +54,8 @@ int ddx_conv3x3(void* stream, int B, int H, int W, int Ci, int Co, const void* x
 /* Weight gradient dw[co][t][ci] = sum_p dz[p][co] x[shift_t(p)][ci] (fp32,
  * padded layout).  partial is scratch of nchunk * Co * 9 * Ci floats; the
  * pixel range is split into at most nchunk chunks whose partial sums are
- * added in a fixed order (deterministic). */
+ * added in a fixed order (deterministic).  The shapes of the LDS-tiled
+ * kernel above take one here too, where x and dz are 8-byte aligned. */
 int ddx_conv3x3_wgrad(void* stream, int B, int H, int W, int Ci, int Co, const void* x,
                       const void* dz, float* partial, int nchunk, float* dw);
 

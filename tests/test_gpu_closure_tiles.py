@@ -59,3 +59,35 @@ def test_gradients(B, H, W, Ci, Co):
         dwp = net.wgrad(xd, dzd, B, H, W, nchunk=nchunk)
         assert rl2(net.wunpack(dwp, Co, Ci), dw) < 1e-5, nchunk
         assert torch.equal(dwp, net.wgrad(xd, dzd, B, H, W, nchunk=nchunk))
+
+
+@pytest.mark.parametrize("B,H,W,Ci,Co", [(1, 8, 32, 32, 32), (1, 4, 64, 16, 32)], ids=str)
+@pytest.mark.parametrize("odd", ["x", "dz"])
+def test_weight_gradient_alignment(B, H, W, Ci, Co, odd):
+    """The tile kernel reads x and dz 8 bytes at a time; arrays that start on
+    another 2-byte boundary go to the per-fragment kernel.  Which one ran shows
+    in the partial sums: a single tile fills one chunk, 64-pixel chunks all four."""
+    import ctypes
+    from dedalus import _hip
+    d, net = dev(), C()
+    case("wgrad alignment", B, H, W, Ci, Co, odd)
+    x, w, _ = random_conv(B, H, W, Ci, Co, 44)
+    dz = torch.randn(B, H, W, Co, generator=torch.Generator().manual_seed(45)).to(torch.bfloat16)
+    _, ref = R.conv_grads(R.nhwc_to_nchw(x.double()), w.double(), R.nhwc_to_nchw(dz.double()))
+
+    def at(t, off):
+        buf = torch.zeros(t.numel() + 8, dtype=torch.bfloat16, device=d)
+        buf[off:off + t.numel()] = t.reshape(-1).to(d)
+        return buf, ctypes.c_void_p(buf.data_ptr() + 2 * off)
+
+    used = {}
+    for off in (0, 4, 1):
+        xb, xp = at(x, off if odd == "x" else 0)
+        db, dp = at(dz, off if odd == "dz" else 0)
+        part = torch.full((4, Co, 9, Ci), float("nan"), device=d)
+        dw = torch.empty((Co, 9, Ci), device=d)
+        _hip._check(_hip._lib.ddx_conv3x3_wgrad(net._stream(), B, H, W, Ci, Co, xp, dp, net._ptr(part), 4, net._ptr(dw)))
+        torch.cuda.synchronize()
+        assert rl2(net.wunpack(dw, Co, Ci), ref) < 1e-5, off
+        used[off] = int((~part.isnan().flatten(1).any(1)).sum())
+    assert used == {0: 1, 4: 1, 1: 4}

@@ -1,6 +1,7 @@
 // Mixed-radix x-row passes; built once per real type and dimension
 // (DDX_MIX_T, DDX_MIX_ND; DDX_MIX_ND = 0: the plain transforms and the
-// dispatch) so that the parts compile side by side.
+// dispatch, 1: the plain transforms within groups) so that the parts compile
+// side by side.
 #include <hip/hip_runtime.h>
 
 #include "ddx_mixed_dev.h"
@@ -11,7 +12,34 @@ template <typename T, int PH, int ND>
 void mix_row_phys_go(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, unsigned blocks, unsigned thr, size_t lds,
                      long nrows);
 
-#if DDX_MIX_ND > 0
+template <typename T, bool GRP>
+void mix_row_plain_go(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, dim3 grid, unsigned thr, size_t lds,
+                      long nrows, int group);
+
+#if DDX_MIX_ND < 2
+
+template <typename T, bool GRP>
+void mix_row_plain_go(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, dim3 grid, unsigned thr, size_t lds,
+                      long nrows, int group) {
+  if (a.mode == ROW_C2R) {
+    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_c2r<T, 4, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_c2r<T, 5, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else hipLaunchKernelGGL((mix_row_c2r<T, 6, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+  } else {
+    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_r2c<T, 4, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_r2c<T, 5, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+    else hipLaunchKernelGGL((mix_row_r2c<T, 6, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
+  }
+}
+
+template void mix_row_plain_go<double, DDX_MIX_ND == 1>(hipStream_t, const RowArgs<double>&, const MixRow&, dim3,
+                                                        unsigned, size_t, long, int);
+template void mix_row_plain_go<float, DDX_MIX_ND == 1>(hipStream_t, const RowArgs<float>&, const MixRow&, dim3,
+                                                       unsigned, size_t, long, int);
+
+#endif
+
+#if DDX_MIX_ND > 1
 
 template <typename T, int PH, int ND>
 void mix_row_phys_go(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, unsigned blocks, unsigned thr, size_t lds,
@@ -28,21 +56,7 @@ DDX_MIX_INST(PH_HYDRO)
 DDX_MIX_INST(PH_BOUSS)
 DDX_MIX_INST(PH_MHD)
 
-#else
-
-template <typename T, bool GRP>
-static void mix_row_plain_go(hipStream_t s, const RowArgs<T>& a, const MixRow& mr, dim3 grid, unsigned thr, size_t lds,
-                             long nrows, int group) {
-  if (a.mode == ROW_C2R) {
-    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_c2r<T, 4, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
-    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_c2r<T, 5, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
-    else hipLaunchKernelGGL((mix_row_c2r<T, 6, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
-  } else {
-    if (mr.RL == 4) hipLaunchKernelGGL((mix_row_r2c<T, 4, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
-    else if (mr.RL == 5) hipLaunchKernelGGL((mix_row_r2c<T, 5, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
-    else hipLaunchKernelGGL((mix_row_r2c<T, 6, GRP>), grid, dim3(thr), lds, s, a, mr, nrows, group);
-  }
-}
+#elif DDX_MIX_ND == 0
 
 template <typename T>
 bool mix_row_launch(hipStream_t s, const RowArgs<T>& a, const MixRow& mr0, long nrows, long group) {

@@ -60,7 +60,6 @@ struct ColArgs {
   int in_rows, in_c;     // in_c < 0: rows are the full axis
   int out_rows, out_c;   // out_c < 0: rows are the full axis
   int ncols;             // columns per slab
-  int W;                 // tile width (columns per workgroup)
   int row_dim, slab_dim; // physical axis (0 x, 1 y, 2 z) of rows / slabs, -1 none
   int nslabs, nfields;   // grid extents (used by the remapped 1D grids)
   int ntiles;            // column tiles per slab
@@ -229,7 +228,7 @@ __global__ void __launch_bounds__(256) row_kernel(const RowArgs<T> a) {
       A[q * nx + m] = mk(va.x - vb.y, va.y + vb.x);
     }
     __syncthreads();
-    X = lds_fft<T, T, 1>(A, B, a.fp, nsin, 1, nx, false, a.tw, tid, nthr);
+    X = lds_fft<T, T, 1>(A, B, a.fp, nsin, 1, nx, a.tw, tid, nthr);
     if (a.mode == ROW_C2R) {
       for (int e = tid; e < a.nin * nx; e += nthr) {
         const int f = e / nx, m = e - f * nx;
@@ -263,7 +262,7 @@ __global__ void __launch_bounds__(256) row_kernel(const RowArgs<T> a) {
     X = Y;
   }
   cpx<T>* Bf = (X == A) ? B : A;
-  cpx<T>* Z = lds_fft<T, T, -1>(X, Bf, a.fp, nsout, 1, nx, false, a.tw, tid, nthr);
+  cpx<T>* Z = lds_fft<T, T, -1>(X, Bf, a.fp, nsout, 1, nx, a.tw, tid, nthr);
   for (int e = tid; e < nsout * a.kxp; e += nthr) {
     const int q = e / a.kxp, k = e - q * a.kxp;
     cpx<T> ra = mk(T(0), T(0)), rb = mk(T(0), T(0));

@@ -37,7 +37,6 @@ bool mix_col_launch(hipStream_t s, ColArgs<T>& a, const MixPlan& mp0, int nslabs
   mp.wshift = 0;
   while ((1 << mp.wshift) < W) ++mp.wshift;
   const int ntiles = (a.ncols + W - 1) / W;
-  a.W = W;
   a.nslabs = nslabs;
   a.nfields = nfields;
   a.ntiles = ntiles;

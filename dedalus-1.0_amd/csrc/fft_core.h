@@ -207,12 +207,11 @@ DDX_HD void stockham_bfly(const cpx<T>* src, cpx<T>* dst, int i, int nb, int p, 
 // Batched in-LDS FFT over `nseq` sequences of length plan.n.  Element e of
 // sequence s lives at buf[s * ss + e * es].  Ping-pongs between A and B;
 // returns the buffer holding the result.  Work is spread over threads
-// tid = 0..nthr-1 (host callers pass tid = 0, nthr = 1).  When seq_fast is
-// set, consecutive threads take consecutive sequences (used when sequences
-// are adjacent in memory, i.e. ss == 1), otherwise consecutive butterflies.
+// tid = 0..nthr-1 (host callers pass tid = 0, nthr = 1), consecutive threads
+// taking consecutive butterflies.
 template <typename T, typename TW, int D>
 DDX_HD cpx<T>* lds_fft(cpx<T>* A, cpx<T>* B, const FftPlan& plan, int nseq, int es, int ss,
-                       bool seq_fast, const cpx<TW>* tw, int tid, int nthr) {
+                       const cpx<TW>* tw, int tid, int nthr) {
   const int n = plan.n;
   int p = 1;
   for (int pass = 0; pass < plan.npass; ++pass) {
@@ -221,9 +220,7 @@ DDX_HD cpx<T>* lds_fft(cpx<T>* A, cpx<T>* B, const FftPlan& plan, int nseq, int 
     const int twstride = n / (p * R);
     const int total = nseq * nb;
     for (int b = tid; b < total; b += nthr) {
-      int s, i;
-      if (seq_fast) { s = b % nseq; i = b / nseq; }
-      else { s = b / nb; i = b - s * nb; }
+      const int s = b / nb, i = b - s * nb;
       const cpx<T>* src = A + s * ss;
       cpx<T>* dst = B + s * ss;
       switch (R) {

@@ -1662,16 +1662,19 @@ int launch_net(const NetArgs& a, hipStream_t s) {
 // unrolled over the four ring positions, which makes every LDS row an
 // immediate offset.
 //
-// What bounds it: VALU issue, about 2400 cycles of a step's 2700 at 2 GHz (8
-// activations of 14.5 issue slots per lane and wavefront, and the addresses).
-// 256 images 64^2: 213 us with the tile kernel, 1.83 times the network's
-// MFMAs; row by row 150 us with two fragments per wavefront and 8 wavefronts
-// per CU, 128 with one and 16, 112 with the last layer's weights in LDS (128
-// registers without spills).
+// What bounds it: VALU issue first, about 1700 cycles of a step's 2750 (8
+// activations of 14.5 issue slots per lane and wavefront, and the addresses),
+// beside 1300 of MFMAs; the barrier of each step keeps either from filling it
+// (wavefronts wait 48 % of their cycles).  256 images 64^2: 213 us with the
+// tile kernel, 1.83 times the network's MFMAs; row by row 150 us with two
+// fragments per wavefront and 8 wavefronts per CU, 128 with one and 16, 112
+// with the last layer's weights in LDS (128 registers without spills).
 //
 // One 16-byte chunk q (8 channels) of pixel p lies at chunk q ^ ((p >> 2) & 3)
-// of the pixel's 64 bytes: the 16 pixels of a fragment read one chunk each
-// from 16 distinct bank groups, for any shift of the fragment.
+// of the pixel's 64 bytes: the 16 pixels of a fragment lie in 16 distinct
+// 16-byte bank groups, for any shift of the fragment.  The counters still
+// show 3.5 conflict cycles per LDS instruction; which accesses take them is
+// not measured.
 //
 // The arithmetic is conv_net_kernel's: the same products in the same order.
 // Rows before a layer's first and after its last are computed from whatever

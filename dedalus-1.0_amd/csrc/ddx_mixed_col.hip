@@ -24,10 +24,11 @@ bool mix_col_launch(hipStream_t s, ColArgs<T>& a, const MixPlan& mp0, int nslabs
   const bool big = (size_t)a.in_rows * a.in_rs + a.ncols >= lim || (size_t)a.out_rows * a.out_rs + a.ncols >= lim;
   // Tile width: 16 columns within 48 KB of LDS (three workgroups per CU),
   // then narrower down to 64 bytes while the launch would leave CUs without a
-  // workgroup.  Eight FP64 columns cost 4 % at 192^3 (60.0 against 57.7 us,
-  // spectral passes); 32 FP32 columns cost 15-30 % (128^3: 20.5 against 15.5
-  // us spectral; 256 members 128^2: 23.6 against 19.9), a third of it lanes
-  // past the last column of 48.
+  // workgroup.  Eight FP64 columns: 192^3 hydro step 700 against 686 us, 1000
+  // members of 32^2 102 against 92, 75x96x120 transforms back 30.9 against
+  // 32.4, most sizes even.  32 FP32 columns: 192^3 step 412 against 403 us,
+  // 160x144x180 292 against 275, 1000 members of 32^2 88 against 79 (lanes
+  // past the last of their 16 columns), smaller grids even.
   const int wmin = 64 / (int)sizeof(cpx<T>);
   int W = 16;
   while (W > 1 && (size_t)n * W * sizeof(cpx<T>) > 49152) W /= 2;

@@ -459,13 +459,15 @@ template <> struct MixIO<PH_MHD, 2>   { static constexpr int NIN = 6, NOUT = 3; 
 // every field's x values of its RL positions, forms the products and starts
 // the r2c in registers, so x-space data never goes through LDS.
 //
-// 192^3 FP64 hydro (6 fields in, 3 out, 340 MB): 143 us against 398 us of the
-// general row kernel, 2.4 TB/s.  VALU issue is busy 45 % of the time (69 k
-// lane-instructions per row, a third of them index arithmetic) and LDS 42 %,
-// in phases that the barriers keep apart, so wavefronts per SIMD set the
-// time: 3 (156 registers) 173 us, 4 152 us, 5 143 us.  The bounds on the
-// registers below are the largest counts without spills that matter (RL 5
-// and 6 of the 10- and 12-field rows spill at three wavefronts).
+// 192^3 FP64 hydro (6 fields in, 3 out, 340 MB): 138 to 146 us on different
+// cards against 398 us of the general row kernel, 2.3 to 2.5 TB/s.  VALU issue is busy 55 % of the time (71 k
+// lane-instructions per row, a third of them index arithmetic), wavefronts
+// wait 55 % of theirs, in phases that six barriers keep apart, so wavefronts
+// per SIMD set the time (one card: 3, at 156 registers, 173 us, 4 152 us, 5
+// 143 us).  The bounds on the registers below
+// are the largest counts without spills that matter (RL 5 and 6 of the 10-
+// and 12-field rows spill at three wavefronts; the 2D hydro row keeps five
+// with 8 bytes spilled).
 template <typename T, int PH, int ND, int RL>
 __global__ void __launch_bounds__(256, (ND == 3 && PH != PH_HYDRO && sizeof(T) == 8)
                                                  ? (RL == 4 ? 3 : 2)

@@ -43,8 +43,8 @@ bool mix_col_plan(int n, MixPlan* p) {
   while (nb < 2) best[nb++] = 1;   // at least a first and a last pass
   // The first pass takes the largest radix up to 12: with two spectral terms
   // a radix-16 butterfly has 32 loads in flight, 215 registers and two
-  // wavefronts per SIMD; with 12 it is 162 and three (192^3 FP64 spectral
-  // passes 71 -> 57 us, plain 35 -> 33 us).
+  // wavefronts per SIMD; with 12 it is 163 and three (192^3 FP64 spectral
+  // passes 71 -> 57 us, plain 35 -> 33 us; with 64-bit offsets 169 and two).
   if (best[0] > 12) {
     int i = 0;
     while (best[i] > 12) ++i;

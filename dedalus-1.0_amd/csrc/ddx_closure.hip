@@ -16,6 +16,7 @@
 // can be checked against a host product.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <type_traits>
@@ -1618,19 +1619,28 @@ __global__ void __launch_bounds__(NT) conv_net_kernel(NetArgs a) {
   net_layers<0, NL, HID, TX, TY, NT>(a, buf0, buf1, wl, b, y0, x0, w0);
 }
 
+// Lets a kernel take this much dynamic LDS; once per device (done: a bit
+// each), from any thread.
+int allow_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done, const char* name) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  const uint64_t bit = dev < 64 ? 1ull << dev : 0;   // beyond: set on each call
+  if (e == hipSuccess && !(done.load(std::memory_order_acquire) & bit)) {
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
+  }
+  if (e != hipSuccess) return ddx::set_error(DDX_ERR_HIP, std::string(name) + " LDS attribute: " + hipGetErrorString(e));
+  return 0;
+}
+
 template <int NL, int HID, int TX, int TY, int NT>
 int launch_net(const NetArgs& a, hipStream_t s) {
   using P = NetPlan<NL, HID, TX, TY>;
   constexpr int lds = P::lds_bytes();
   static_assert(lds <= 160 * 1024, "tile does not fit the LDS");
-  static bool attr = false;
-  if (!attr) {
-    const hipError_t e = hipFuncSetAttribute((const void*)conv_net_kernel<NL, HID, TX, TY, NT>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess)
-      return ddx::set_error(DDX_ERR_HIP, std::string("conv_net LDS attribute: ") + hipGetErrorString(e));
-    attr = true;
-  }
+  static std::atomic<uint64_t> done{0};
+  const int rc = allow_lds((const void*)conv_net_kernel<NL, HID, TX, TY, NT>, lds, done, "conv_net");
+  if (rc) return rc;
   const long ntiles = (long)a.B * (a.H / TY) * (a.W / TX);
   hipLaunchKernelGGL((conv_net_kernel<NL, HID, TX, TY, NT>), dim3((unsigned)ntiles), dim3(NT), lds, s, a);
   CL_LAUNCHCHK("conv_net");
@@ -1923,14 +1933,9 @@ int launch_rows(const NetArgs& a, int S, hipStream_t s) {
   using P = RowNet<W>;
   constexpr int lds = P::lds_bytes();
   static_assert(lds * P::WG_PER_CU <= 160 * 1024, "rings do not fit the LDS");
-  static bool attr = false;
-  if (!attr) {
-    const hipError_t e = hipFuncSetAttribute((const void*)conv_rows_kernel<W>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess)
-      return ddx::set_error(DDX_ERR_HIP, std::string("conv_rows LDS attribute: ") + hipGetErrorString(e));
-    attr = true;
-  }
+  static std::atomic<uint64_t> done{0};
+  const int rc = allow_lds((const void*)conv_rows_kernel<W>, lds, done, "conv_rows");
+  if (rc) return rc;
   const int strips = (a.H + S - 1) / S;
   hipLaunchKernelGGL((conv_rows_kernel<W>), dim3((unsigned)(a.B * strips)), dim3(P::NT), lds, s, a, S, strips);
   CL_LAUNCHCHK("conv_rows");

@@ -27,7 +27,7 @@ FLAGS = [
 
 # translation units: (source, definitions); compiled side by side and linked
 MIX_ROW = [("double", 0), ("double", 1), ("double", 2), ("double", 3), ("float", 2), ("float", 3)]
-UNITS = [("ddx.hip", []), ("ddx_closure.hip", []), ("ddx_mixed_plan.hip", []),
+UNITS = [("ddx.hip", []), ("ddx_closure.hip", []), ("ddx_mixed_plan.hip", []), ("ddx_row_group.hip", []),
          ("ddx_mixed_col.hip", ["-DDDX_MIX_T=double"]), ("ddx_mixed_col.hip", ["-DDDX_MIX_T=float"])] + [
     ("ddx_mixed_row.hip", ["-DDDX_MIX_T=%s" % t, "-DDDX_MIX_ND=%d" % nd]) for t, nd in MIX_ROW]
 

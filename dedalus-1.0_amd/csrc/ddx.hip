@@ -561,8 +561,9 @@ void row_plain_nv(ddx_plan* p, const RowArgs<T>& a, long nrows) {
   const long teams = group ? nrows / group * ((group + 1) / 2) : (nrows + 1) / 2;
   const int nf = a.mode == ROW_C2R ? a.nin : a.nout;   // grid.y: the field
   const dim3 grid((unsigned)((teams + RPB - 1) / RPB), (unsigned)nf);
-  if (a.mode == ROW_C2R) hipLaunchKernelGGL((row_c2r_fast<T, N, V>), grid, dim3(64), 0, p->stream, a, nrows, group);
-  else hipLaunchKernelGGL((row_r2c_fast<T, N, V>), grid, dim3(64), 0, p->stream, a, nrows, group);
+  if (group) row_group_go<T, N, V>(p->stream, a, nrows, group, grid);
+  else if (a.mode == ROW_C2R) hipLaunchKernelGGL((row_c2r_fast<T, N, V, false>), grid, dim3(64), 0, p->stream, a, nrows, 0);
+  else hipLaunchKernelGGL((row_r2c_fast<T, N, V, false>), grid, dim3(64), 0, p->stream, a, nrows, 0);
 }
 
 template <typename T, int N>

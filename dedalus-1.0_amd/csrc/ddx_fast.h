@@ -500,13 +500,19 @@ __global__ void __launch_bounds__(64) row_phys_fast(const RowArgs<T> a, long nro
 
 // ---------------------------------------------------------------------------
 // plain x-row transforms (ddx_bwd / ddx_fwd): two rows of one field per team,
-// the field (of several in one call) in blockIdx.y
+// the field (of several in one call) in blockIdx.y; GRP: pairs stay inside
+// groups of rows (row_pair)
 // ---------------------------------------------------------------------------
+
+// Launches the grouped forms, which are built in a unit of their own
+// (ddx_row_group.hip)
+template <typename T, int N, int V>
+void row_group_go(hipStream_t s, const RowArgs<T>& a, long nrows, int group, dim3 grid);
 
 // c2r of rows 2t and 2t + 1: z = A + i B from the two half spectra, one
 // inverse transform, x rows = (Re z, Im z).  Loads as in row_phys_fast
 // (clamped addresses, zeroed afterwards, the k = 0 imaginary part dropped).
-template <typename T, int N, int V = 0>
+template <typename T, int N, int V, bool GRP>
 __global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrows, int group) {
   using PL = RowPlanV<N, V>;
   constexpr int LANES = PL::LANES, E = PL::E, RPB = 64 / LANES;
@@ -517,7 +523,7 @@ __global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrow
   const int team = threadIdx.x / LANES, lane = threadIdx.x % LANES;
   long ra;
   bool live_a, live_b;
-  row_pair((long)blockIdx.x * RPB + team, nrows, group, ra, live_a, live_b);
+  row_pair((long)blockIdx.x * RPB + team, nrows, GRP ? group : 0, ra, live_a, live_b);
   const long la_row = live_a ? ra : nrows - 1, lb_row = live_b ? ra + 1 : nrows - 1;
   const int cx = a.kx - 1;
   cpx<T> twc[PL::NP][E];
@@ -565,7 +571,7 @@ __global__ void __launch_bounds__(64) row_c2r_fast(const RowArgs<T> a, long nrow
 // r2c of rows 2t and 2t + 1: z = a + i b, one forward transform, half
 // spectra A = (Z_k + conj Z_{N-k}) / 2, B = (Z_k - conj Z_{N-k}) / 2i.  The
 // x loads sit at the first-pass positions of the reversed radix order.
-template <typename T, int N, int V = 0>
+template <typename T, int N, int V, bool GRP>
 __global__ void __launch_bounds__(64) row_r2c_fast(const RowArgs<T> a, long nrows, int group) {
   using PL = RowPlanV<N, V>;
   constexpr int LANES = PL::LANES, E = PL::E, RPB = 64 / LANES;
@@ -577,7 +583,7 @@ __global__ void __launch_bounds__(64) row_r2c_fast(const RowArgs<T> a, long nrow
   const int team = threadIdx.x / LANES, lane = threadIdx.x % LANES;
   long ra;
   bool live_a, live_b;
-  row_pair((long)blockIdx.x * RPB + team, nrows, group, ra, live_a, live_b);
+  row_pair((long)blockIdx.x * RPB + team, nrows, GRP ? group : 0, ra, live_a, live_b);
   const long la_row = live_a ? ra : nrows - 1, lb_row = live_b ? ra + 1 : nrows - 1;
   cpx<T>* buf = lds[team];
   cpx<T> twf[PL::NP][E];

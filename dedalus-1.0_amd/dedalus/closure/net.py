@@ -192,20 +192,37 @@ def unpack(src, C, dsts, f64, pstride=1, scale=None, add=None):
                                1 if f64 else 0, sc, ad))
 
 
-def _param(p, shape, dev):
+def _param(p, shape, dev, co=None):
     """A parameter as the contiguous float32 tensor of this shape that the
-    kernels read: a smaller weight is padded with zeros, a bias broadcast."""
+    kernels read: a weight is padded with zeros or cut, a bias broadcast to its
+    layer's co channels and padded."""
     if p.shape == shape and p.dtype == torch.float32 and p.device == dev and p.is_contiguous():
         return p
     p = p.detach().to(device=dev, dtype=torch.float32)
-    if p.shape != shape:
-        if len(shape) == 1:
-            p = p.expand(shape)
-        elif p.dim() != 4 or p.shape[2:] != (3, 3) or p.shape[0] > shape[0] or p.shape[1] > shape[1]:
-            raise ValueError("closure weights of shape %s do not fit a layer of %s" % (tuple(p.shape), shape))
-        else:
-            p = torch.nn.functional.pad(p, (0, 0, 0, 0, 0, shape[1] - p.shape[1], 0, shape[0] - p.shape[0]))
+    if len(shape) == 1:
+        p = p.expand((shape[0] if co is None else co,))
+    else:
+        p = p[:shape[0], :shape[1]]
+        p = torch.nn.functional.pad(p, (0, 0, 0, 0, 0, shape[1] - p.shape[1]))
+    if p.shape[0] != shape[0]:
+        p = torch.nn.functional.pad(p, (0, 0) * (p.dim() - 1) + (0, shape[0] - p.shape[0]))
     return p.contiguous()
+
+
+def _widths(chans, ws):
+    """Channels per layer including those that weights larger than their layer
+    bring in its padding: a hidden layer computes them, and the next one uses
+    them where its weights reach that far."""
+    full = list(chans)
+    for l, w in enumerate(ws):
+        if w.dim() != 4 or w.shape[2:] != (3, 3) or w.shape[0] > pad16(chans[l + 1]) or w.shape[1] > pad16(chans[l]):
+            raise _hip.DDXError(-1, "closure weights of shape %s do not fit a layer of %d channels from %d"
+                                % (tuple(w.shape), chans[l + 1], chans[l]))
+        if l < len(ws) - 1:
+            full[l + 1] = max(full[l + 1], w.shape[0])
+        if l > 0:
+            full[l] = max(full[l], w.shape[1])
+    return full
 
 
 def _chans(chans):
@@ -224,19 +241,24 @@ class _NetFn(torch.autograd.Function):
         assert cin == chans[0] and B * H * W % 16 == 0
         lib = _lib()
         dev = x.device
-        ch = _chans(chans)
+        full = chans
+        for l in range(nl):
+            if params[l].shape != (chans[l + 1], chans[l], 3, 3):
+                full = _widths(chans, params[:nl])
+                break
+        ch = _chans(full)
         nsaved, nscratch = ctypes.c_int64(), ctypes.c_int64()
         _check(lib.ddx_net_bytes(B, H, W, nl, ch, nsaved, nscratch))
         xc = x.detach().contiguous()
-        ws = [_param(params[l], (chans[l + 1], chans[l], 3, 3), dev) for l in range(nl)]
-        bs = [_param(params[nl + l], (chans[l + 1],), dev) for l in range(nl)]
+        ws = [_param(params[l], (full[l + 1], full[l], 3, 3), dev) for l in range(nl)]
+        bs = [_param(params[nl + l], (full[l + 1],), dev, chans[l + 1]) for l in range(nl)]
         saved = torch.empty(nsaved.value, dtype=torch.uint8, device=dev)
         out = torch.empty((B, H, W, chans[-1]), dtype=torch.float32, device=dev)
         _check(lib.ddx_net_forward(_stream(), B, H, W, nl, ch, _ptr(xc),
                                    _hip.ptr_array([p.data_ptr() for p in ws]),
                                    _hip.ptr_array([p.data_ptr() for p in bs]),
                                    _ptr(saved), _ptr(out)))
-        ctx.chans = chans
+        ctx.chans, ctx.full = chans, full
         ctx.shape = (B, H, W)
         ctx.nscratch = nscratch.value
         ctx.save_for_backward(saved)
@@ -244,7 +266,7 @@ class _NetFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        chans = ctx.chans
+        chans, full = ctx.chans, ctx.full
         nl = len(chans) - 1
         B, H, W = ctx.shape
         saved, = ctx.saved_tensors
@@ -253,12 +275,15 @@ class _NetFn(torch.autograd.Function):
         gc = g.detach().contiguous()
         dev = gc.device
         scratch = torch.empty(ctx.nscratch, dtype=torch.uint8, device=dev)
-        gws = [torch.empty((chans[l + 1], chans[l], 3, 3), dtype=torch.float32, device=dev)
+        gws = [torch.empty((full[l + 1], full[l], 3, 3), dtype=torch.float32, device=dev)
                for l in range(nl)]
-        gbs = [torch.empty(chans[l + 1], dtype=torch.float32, device=dev) for l in range(nl)]
-        _check(_lib().ddx_net_backward(_stream(), B, H, W, nl, _chans(chans), _ptr(gc), _ptr(saved),
+        gbs = [torch.empty(full[l + 1], dtype=torch.float32, device=dev) for l in range(nl)]
+        _check(_lib().ddx_net_backward(_stream(), B, H, W, nl, _chans(full), _ptr(gc), _ptr(saved),
                                        _ptr(scratch), _hip.ptr_array([t.data_ptr() for t in gws]),
                                        _hip.ptr_array([t.data_ptr() for t in gbs])))
+        if full is not chans:
+            gws = [g[:chans[l + 1], :chans[l]] for l, g in enumerate(gws)]
+            gbs = [g[:chans[l + 1]] for l, g in enumerate(gbs)]
         return (None, None, *gws, *gbs)
 
 

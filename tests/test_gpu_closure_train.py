@@ -75,3 +75,36 @@ def test_network_calls_match_layers(shape, chans):
         assert torch.equal(net.weights[l].grad, gw[l]), l
         bound = 2.0 ** -23 * gb[l].double().abs() + npix * 2.0 ** -53 * mag[l] + 1e-40
         assert ((net.biases[l].grad.double() - gb[l].double()).abs() <= bound).all(), l
+
+
+def test_weights_larger_than_their_layers():
+    """Weights within a layer's padding of 16 but beyond its channels compute
+    the extra channels, which the next layer's weights may read; beyond the
+    padding they are refused.  Smaller ones count as zeros there."""
+    from dedalus import _hip
+    from dedalus.closure import ClosureNet
+    from dedalus.closure import net as N
+    print("net calls, other weight shapes", flush=True)
+    d = torch.device("cuda")
+    gen = torch.Generator().manual_seed(22)
+    chans = (3, 20, 20, 2)
+    net = ClosureNet(cin=3, cout=2, width=20, depth=3, seed=3, out_scale=1.0).to(d)
+
+    def put(shapes):
+        for l, (co, ci) in enumerate(shapes):
+            net.weights[l] = torch.nn.Parameter((torch.randn(co, ci, 3, 3, generator=gen) * 0.2).to(d))
+            net.biases[l] = torch.nn.Parameter((torch.randn(chans[l + 1], generator=gen) * 0.1).to(d))
+
+    x = torch.randn(2, 8, 64, 3, generator=gen).to(d)
+    g = torch.randn(2, 8, 64, 2, generator=gen).to(d)
+    for shapes in ([(24, 5), (20, 26), (3, 20)], [(18, 3), (20, 16), (1, 20)]):
+        put(shapes)
+        with torch.no_grad():
+            out = net(x)
+        ref = layer_calls(N, x, g, chans, [w.detach() for w in net.weights], [b.detach() for b in net.biases])[0]
+        assert torch.equal(out, ref), shapes
+        with pytest.raises(RuntimeError):       # their gradient has the layer's shape
+            net(x).backward(g)
+    put([(20, 3), (33, 20), (2, 20)])
+    with pytest.raises(_hip.DDXError):
+        net(x)
